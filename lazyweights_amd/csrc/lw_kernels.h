@@ -148,7 +148,7 @@ constexpr int TILES_ROWC = 64;
 hipError_t launch_fused_halves(const FlatPlan& plan, int per, hipStream_t s);
 int halves_buf_rows(const FlatPlan& plan);
 int tiles_buf_rows(const FlatPlan& plan);
-// The whole-tile kernel for 2..8 tokens of fp16 activations (every format, plan.mt tokens, every tile of each entry):
+// The whole-tile kernel for 2..4 tokens of fp16 activations (every format, plan.mt tokens, every tile of each entry):
 // the products on the matrix cores (4x4x4 blocks, x broadcast from one block), every token in one pass over the
 // tiles; each block forms the x sums of its tile columns in LDS (tiles_mma_xs_bytes beside W tile buffers of
 // tiles_buf_rows word rows)
@@ -158,6 +158,43 @@ size_t tiles_mma_xs_bytes(const FlatPlan& plan, int per);
 // launch_quant_x8): integer products on the matrix cores per sub-block, folded with the block scales in fp32
 hipError_t launch_fused_tiles_mma8(const FlatPlan& plan, int per, hipStream_t s);
 int tiles_mma_max_waves(int kqt, int mt);  // the block limit of both matrix-core whole-tile kernels
+
+// The 16-token kernel (lw_wide.hip): mt <= 16 pseudo-tokens of fp16 activations (per = 2: fp32 activations as hi + lo
+// rows, mt / 2 tokens out), any mix of formats, blocks of W waves with half a tile each. Entry i owns wide_blocks(M, w)
+// blocks from block0, at most w units (half tiles) each; w a multiple of 4 unless KT <= w, so that a matrix's results do
+// not depend on it. X: launch_wide_x's output. Y rows ldy apart; P: KT mt N partial slots (kNoPartial outside a launch),
+// cnt: 2 NT zeroed counters (left zeroed).
+struct WideEntry {
+  DevMat M;
+  const void* X;
+  float* P;
+  float* Y;
+  uint32_t* cnt;
+  int ldy;
+  int block0, w;
+};
+struct WidePlan {
+  WideEntry e[MAX_GROUP];
+  int n, W, mt, per;
+};
+constexpr int WIDE_MAX_WAVES = 16;
+size_t wide_x_bytes(int mt, int K);  // bytes of one reordered vector
+// activations for it in one launch: job i reorders X[i] (fp16 [mt][K], any alignment; per = 2: fp32 [mt / 2][K], split
+// into hi + lo) into XT[i] (mt K fp16, 16-byte aligned)
+struct WideXJobs {
+  const void* X[MAX_GROUP];
+  void* XT[MAX_GROUP];
+  int K[MAX_GROUP];
+  int symbits[MAX_GROUP];
+  int b0[MAX_GROUP];  // set by the launch
+  int n, mt, per;
+};
+hipError_t launch_wide_x(WideXJobs q, hipStream_t s);
+bool wide_ok(const DevMat& M);
+int wide_blocks(const DevMat& M, int w);
+int wide_buf_rows(const WidePlan& plan);
+size_t wide_lds_bytes(int waves, int buf_rows);
+hipError_t launch_fused_wide(const WidePlan& plan, hipStream_t s);
 
 // One launch of the ring kernel over all matrices of the plan (returns hipErrorInvalidValue if the plan mixes
 // K-quant types or ring sizes, or a matrix has no ring schedule).

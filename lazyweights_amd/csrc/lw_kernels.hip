@@ -14,24 +14,9 @@
 //     once per sub-block;
 //   * partial sums per tile column go to P[tc][j][n] and are summed in tile-column order by k_reduce
 //     (deterministic, as the reference's k_sum_kt, llmrt.cu:1171-1180).
-#include <hip/hip_runtime.h>
-#include <type_traits>
-
-#include "lw_format.h"
-#include "lw_kernels.h"
+#include "lw_device.h"
 
 namespace lw {
-
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-
-// leading zero bits of every device lane stream (lw_layout.h GUARD)
-constexpr int GUARD_BITS = 2;
-constexpr int kBufferRsrcWord3 = 0x00020000;  // buffer descriptor word 3 for raw dword loads on CDNA (32-bit data format)
-
-typedef _Float16 h4v __attribute__((ext_vector_type(4)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef int v4i32 __attribute__((ext_vector_type(4)));
-typedef float f16x16 __attribute__((ext_vector_type(16)));
 
 // Activations of MT pseudo-tokens staged in LDS as fp16 pairs: pair c (weights 2c, 2c + 1) of token j. With
 // MT >= 4 (the MFMA path) the two pairs of one 4-weight step are adjacent per token, so a lane reads its token's
@@ -44,11 +29,6 @@ __device__ __forceinline__ int xs_index(int c, int j) {
 __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   return __builtin_amdgcn_fdot2(__builtin_bit_cast(h2v, a), __builtin_bit_cast(h2v, b), c, false);
 }
-__device__ __forceinline__ float h2f(uint32_t bits16) {
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)(bits16 & 0xFFFFu));
-}
-__device__ __forceinline__ uint32_t f2h(float v) { return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v); }
-
 // grid value f(q) of a code (reference llmrt.cu:151-154): Q4_K/Q5_K q, Q6_K q - 32, IQ4_XS kv[q]
 template <int KQ>
 __device__ __forceinline__ float grid_value(uint32_t q) {
@@ -56,28 +36,6 @@ __device__ __forceinline__ float grid_value(uint32_t q) {
   if (KQ == KQ_Q6_K) return (float)q - 32.f;
   return (float)q;
 }
-
-// side bytes of one super-block as words (byte i at bits 8 (i & 3) of w[i / 4]); Q6_K records are 2-byte aligned
-template <int KQ>
-__device__ __forceinline__ void side_load(const uint8_t* p, uint32_t* w) {
-  if (KQ == KQ_Q6_K) {
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) w[i] = (uint32_t)h[2 * i] | (uint32_t)h[2 * i + 1] << 16;
-    w[4] = h[8];
-  } else if (KQ == KQ_IQ4_XS) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    w[0] = v.x;
-    w[1] = v.y;
-  } else {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    w[0] = v.x;
-    w[1] = v.y;
-    w[2] = v.z;
-    w[3] = v.w;
-  }
-}
-__device__ __forceinline__ uint32_t side_byte(const uint32_t* w, int i) { return (w[i >> 2] >> (8 * (i & 3))) & 255u; }
 
 // (s, o) of sub-block j (reference llmrt.cu:125-149; llama.cpp get_scale_min_k4 for Q4_K/Q5_K)
 template <int KQ>
@@ -100,48 +58,6 @@ __device__ __forceinline__ void side_scale(const uint32_t* w, int j, float& s, f
     const uint32_t ls = ((side_byte(w, 4 + j / 2) >> (4 * (j & 1))) & 15) | (((w[0] >> (16 + 2 * j)) & 3) << 4);
     s = h2f(w[0]) * (float)((int)ls - 32);
     o = 0.f;
-  }
-}
-
-// Sub-block scales of one super-block packed as bytes, consumed low byte first (reference llmrt.cu:125-149; Q4_K /
-// Q5_K fields per llama.cpp get_scale_min_k4, four at a time): s_j = dA * byte_j (Q6_K: signed bytes, 16 of them in
-// scq then scq2; IQ4_XS: ls_j - 32, also signed), o_j = dB * m_j (side_mins).
-template <int KQ>
-__device__ __forceinline__ void side_packed(const uint32_t* w, uint64_t& scq, uint64_t& scq2, float& dA, float& dB) {
-  if (KQ == KQ_Q4_K || KQ == KQ_Q5_K) {
-    const uint32_t sc_lo = w[1] & 0x3F3F3F3Fu;
-    const uint32_t sc_hi = (w[3] & 0x0F0F0F0Fu) | ((w[1] >> 2) & 0x30303030u);
-    scq = (uint64_t)sc_lo | (uint64_t)sc_hi << 32;
-    scq2 = 0;
-    dA = h2f(w[0]);
-    dB = h2f(w[0] >> 16);
-  } else if (KQ == KQ_Q6_K) {
-    scq = (uint64_t)w[0] | (uint64_t)w[1] << 32;
-    scq2 = (uint64_t)w[2] | (uint64_t)w[3] << 32;
-    dA = h2f(w[4]);
-    dB = 0.f;
-  } else {
-    const uint32_t hi = w[0] >> 16, lo = w[1];
-    uint64_t q = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t ls = ((lo >> (4 * i)) & 15u) | (((hi >> (2 * i)) & 3u) << 4);
-      q |= (uint64_t)((ls - 32u) & 255u) << (8 * i);
-    }
-    scq = q;
-    scq2 = 0;
-    dA = h2f(w[0]);
-    dB = 0.f;
-  }
-}
-// Q4_K / Q5_K sub-block mins as floats
-__device__ __forceinline__ void side_mins(const uint32_t* w, float* mf) {
-  const uint32_t m_lo = w[2] & 0x3F3F3F3Fu;
-  const uint32_t m_hi = ((w[3] >> 4) & 0x0F0F0F0Fu) | ((w[2] >> 2) & 0x30303030u);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    mf[i] = (float)((m_lo >> (8 * i)) & 255u);
-    mf[4 + i] = (float)((m_hi >> (8 * i)) & 255u);
   }
 }
 
@@ -377,33 +293,11 @@ struct RingStager {
 // used (ring slot and bit offset), and the entries' upper halves only disturb bits >= 16.
 // block = WPB tile rows of one tile column of one matrix of the plan.
 
-// LDS address of the table entry indexed by window bits 2..12 of w: (w & 0x1FFC) | table base, one instruction (the
-// base is a multiple of 8 KB and wave-uniform)
-__device__ __forceinline__ uint32_t table_addr(uint32_t w, uint32_t base, uint32_t mask) {
-  uint32_t a;  // VOP3 takes no literal here: the mask 0x1FFC lives in a register
-  asm("v_and_or_b32 %0, %1, %3, %2" : "=v"(a) : "v"(w), "s"(base), "v"(mask));
-  return a;
-}
-
 // LDS address of the entry of the code at window bits 2..12 of w by the comparator lookup (reference
 // hw/huff/huff_engine.h:54-77) over a matrix's comparator table (canon_table): v = the 11 window bits with the
 // code's first bit most significant; its length l is 1 + the number of limits lim[0..9] that v reaches, and
 // pk[l - 1] = (table base + 4 (base_l - first_l)) << 16 | (11 - l) turns v into the entry's address. lim and pk
 // are wave-uniform (SGPRs): 10 subtract / shift / insert steps per code.
-// compile-time loop: f(std::integral_constant<int, i>) for i = 0 .. N - 1 (indices that must be constants: MFMA
-// broadcast fields, register-array indices; bodies past the loop unroller's size limit)
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for_from(F& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for_from<I + 1, N>(f);
-  }
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_from<0, N>(f);
-}
-
 __device__ __forceinline__ uint32_t canon_addr(uint32_t w, const uint32_t* lim, const uint32_t* pk) {
   const uint32_t v = __builtin_amdgcn_ubfe(__builtin_bitreverse32(w), 19, 11);
   uint32_t p = pk[0];
@@ -814,39 +708,6 @@ __global__ void __launch_bounds__(WPB * 64, MT <= 2 ? 8 : (MT <= 8 ? 4 : 2)) k_f
 // (reduced by a separate launch, which resets the slots likewise). Slots start as kNoPartial (filled when the
 // partials buffer is allocated).
 
-// The sum over columns c < KT, in order, of the partial slots q + c cs. Each slot is taken by an exchange with
-// kNoPartial, 32 in flight. A slot still holding kNoPartial (its partial counted but not yet visible here) makes the
-// running sum NaN, so one test per batch finds it; the batch is then summed again once every such slot has its
-// partial (at most kPartialSpins re-reads each, a few hundred cycles apiece; past that the sum is NaN rather than a
-// hang). A NaN of the data itself only costs the re-summation: no arithmetic result has kNoPartial's bits.
-__device__ __forceinline__ float sum_partials(uint32_t* q, size_t cs, int KT) {
-  constexpr int B = 32;
-  auto take = [&](int c) {
-    return __hip_atomic_exchange(q + (size_t)c * cs, kNoPartial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  float a = 0.f;
-  for (int c0 = 0; c0 < KT; c0 += B) {
-    uint32_t v[B];
-#pragma unroll
-    for (int u = 0; u < B; ++u) v[u] = c0 + u < KT ? take(c0 + u) : 0u;
-    const float a0 = a;
-#pragma unroll
-    for (int u = 0; u < B; ++u)
-      if (c0 + u < KT) a += __builtin_bit_cast(float, v[u]);
-    if (__builtin_expect(a != a, 0)) {
-      a = a0;
-      for (int u = 0; u < B && c0 + u < KT; ++u) {
-        uint32_t w = v[u];
-        for (int i = 0; w == kNoPartial && i < kPartialSpins; ++i) {
-          __builtin_amdgcn_s_sleep(2);
-          w = take(c0 + u);
-        }
-        a += w == kNoPartial ? __builtin_nanf("") : __builtin_bit_cast(float, w);
-      }
-    }
-  }
-  return a;
-}
 // The sums of tile row tr's partials, per token j < mt, by the wave that counted the row's last tile (it also resets
 // the counter). P is [KT][mt][N]: token j's partial of tile column c at P + (c mt + j) N.
 // (reset = false: the row was counted elsewhere, its counter is untouched)
@@ -1634,19 +1495,6 @@ __device__ __forceinline__ void dot2_row(float& acc, uint32_t xrow, int k, uint3
     case 13: dot2_bcast<13>(acc, xrow, w); break;
     case 14: dot2_bcast<14>(acc, xrow, w); break;
     default: dot2_bcast<15>(acc, xrow, w); break;
-  }
-}
-
-// s_waitcnt vmcnt(n) for a wave-uniform n in [0, 63] (the count is an immediate: one wait per value; larger n wait
-// for 63). The compiler does not see which value ran, so it still waits for every vector load whose result a later
-// instruction reads; this is for loads whose results only LDS reads see (direct-to-LDS copies).
-template <int N = 63>
-__device__ __forceinline__ void wait_vmcnt_upto(int n) {
-  if constexpr (N == 0) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  } else {
-    if (n >= N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-    else wait_vmcnt_upto<N - 1>(n);
   }
 }
 
@@ -2551,7 +2399,7 @@ k_fused_halves(FlatPlan plan, int per, int ubuf_rows) {
   reduce_pending();
 }
 
-// ── whole-tile kernel on the matrix cores (2..8 tokens, fp16 activations, every format) ───────────────────
+// ── whole-tile kernel on the matrix cores (2..4 tokens, fp16 activations, every format) ───────────────────
 // The decode of k_fused_tiles (a tile per wave in LDS; 4 chains per lane), with the products of MT tokens on
 // v_mfma_f32_4x4x4f16 (16 blocks of 4 lanes): block b computes D[i][j] = sum_k A[4 b' + i][k] B[4 b + j][k] into lane
 // 4 b + j, register i, where b' is the block named by the instruction's broadcast field (cbsz 4, abid b'). B = the
@@ -2583,7 +2431,7 @@ __global__ void __launch_bounds__(64 * (tiles_mma_waves(KQA, MT) < tiles_mma_wav
                                                                                          : tiles_mma_waves(KQB, MT)),
                                   1)
 k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
-  static_assert(MT == 4 || MT == 8, "4 or 8 token slots");
+  static_assert(MT == 4, "4 token slots");
   constexpr int NQ = MT / 4;      // token quads
   constexpr int NC = 4, NG = 16 / NC;  // chains per lane (64 symbols each: 8 tokens' x and accumulators leave no
                                        // registers for 8 chains at 4 waves per SIMD), 16-symbol groups per chain
@@ -3024,8 +2872,7 @@ static hipError_t tiles_mma_launch_t(const FlatPlan& p, int per, int buf_rows, h
 // two K-quant types in one launch: entries [0, nfa) of type KQA < KQB, the rest of KQB
 template <int KQA, int KQB>
 static hipError_t tiles_mma_launch_mixed_t(const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
-  return p.mt <= 4 ? tiles_mma_launch_t<KQA, 2, 4, KQB>(p, per, buf_rows, s)
-                   : tiles_mma_launch_t<KQA, 2, 8, KQB>(p, per, buf_rows, s);
+  return tiles_mma_launch_t<KQA, 2, 4, KQB>(p, per, buf_rows, s);
 }
 static hipError_t tiles_mma_launch_mixed(int kqa, int kqb, const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
   switch (kqa * 8 + kqb) {
@@ -3041,9 +2888,7 @@ static hipError_t tiles_mma_launch_mixed(int kqa, int kqb, const FlatPlan& p, in
 
 template <int KQ>
 static hipError_t tiles_mma_launch(const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
-  const bool one = p.n == 1;
-  if (p.mt <= 4) return one ? tiles_mma_launch_t<KQ, 1, 4>(p, per, buf_rows, s) : tiles_mma_launch_t<KQ, 2, 4>(p, per, buf_rows, s);
-  return one ? tiles_mma_launch_t<KQ, 1, 8>(p, per, buf_rows, s) : tiles_mma_launch_t<KQ, 2, 8>(p, per, buf_rows, s);
+  return p.n == 1 ? tiles_mma_launch_t<KQ, 1, 4>(p, per, buf_rows, s) : tiles_mma_launch_t<KQ, 2, 4>(p, per, buf_rows, s);
 }
 
 // ── whole-tile kernel on the matrix cores for int8 activations (2..8 tokens, every format) ─────────────────
@@ -3566,7 +3411,7 @@ hipError_t launch_fused_tiles_mma8(const FlatPlan& p, int per, hipStream_t s) {
 }
 
 hipError_t launch_fused_tiles_mma(const FlatPlan& p, int per, hipStream_t s) {
-  if (p.n < 1 || p.n > MAX_GROUP || p.W < 1 || per < p.W || p.ntiles < 1 || p.mt < 1 || p.mt > 8 || p.i8)
+  if (p.n < 1 || p.n > MAX_GROUP || p.W < 1 || per < p.W || p.ntiles < 1 || p.mt < 1 || p.mt > 4 || p.i8)
     return hipErrorInvalidValue;
   // two K-quant types: entries [0, nfa) of the first (the smaller type code), the rest of the second
   const bool mixed = p.nfa > 0 && p.nfa < p.n;
@@ -4330,9 +4175,6 @@ hipError_t launch_gemm_codes_mfma(const DevMat& M, const uint8_t* codes, int row
 // takes super-blocks w, w + GEMM_WAVES, ...) and their partial tiles are summed through LDS in wave order, so the
 // result does not depend on timing. A skinny prefill (m = 128, N = 4096) gives 256 blocks.
 constexpr int GEMM_WAVES = 8;
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 // codes q0..q3 (bytes of qw) -> sc q / 16 as 4 fp16 in two words (nsc = -64 sc)
 __device__ __forceinline__ uint2 scaled_codes16(uint32_t qw, h2v sc, h2v nsc) {
   const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x54545454u, qw, 0x04010400u));

@@ -119,6 +119,8 @@ struct Model {
   size_t cnt_cap = 0;
   uint16_t* X16 = nullptr;
   size_t X16_cap = 0;
+  uint8_t* XW = nullptr;  // activations in the 16-token kernel's order (launch_wide_x)
+  size_t XW_cap = 0;
   uint16_t* SX = nullptr;  // per-sub-block activation sums (prefill GEMM)
   size_t SX_cap = 0;
   uint8_t* x8 = nullptr;  // int8 activations: per vector [K int8][K / 32 d][K / 32 d sum q], 256-B aligned parts
@@ -440,6 +442,7 @@ void release(Model* M) {
   if (M->P) (void)hipFree(M->P);
   if (M->cnt) (void)hipFree(M->cnt);
   if (M->X16) (void)hipFree(M->X16);
+  if (M->XW) (void)hipFree(M->XW);
   if (M->SX) (void)hipFree(M->SX);
   if (M->x8) (void)hipFree(M->x8);
   if (M->codes) (void)hipFree(M->codes);
@@ -548,6 +551,7 @@ struct X8 {
 struct FixedScratch {
   uint8_t* base;
   size_t bytes;
+  uint16_t* x16 = nullptr;  // fp32 activations: room for them as fp16 hi + lo rows
 };
 
 // Quantize the activations of each of `count` matrices (m tokens [m][K_i], fp16 or fp32; a vector shared by several
@@ -622,7 +626,8 @@ int tiles_width(const lw::FlatPlan& fp, int mintiles, int& per) {
   return std::min(wmax, (per + rounds - 1) / rounds);
 }
 
-// Waves per block and tiles per block of the matrix-core whole-tile kernel (2..8 tokens): the tiles as tiles_width,
+// Waves per block and tiles per block of the matrix-core whole-tile kernels (2..4 tokens of fp16, 2..8 of int8
+// activations): the tiles as tiles_width,
 // each block's x sums (tiles_mma_xs_bytes) beside the tile buffers, and as many waves as the LDS holds (measured at
 // m = 2..8 on config 2: 12 waves taking 26 tiles in rounds of 12, 12 and 2 ran 6-9 % faster than 9 waves in 3
 // rounds, unlike the m = 1 kernel). Returns 0 if no width fits.
@@ -654,16 +659,52 @@ int halves_width(const lw::FlatPlan& fp, int mintiles, int& per) {
   return std::min(wmax, 2 * per);
 }
 
-// Fused GEMV / skinny GEMM of `count` matrices with fp16 activations X16[i] ([m * per][K_i] pseudo-tokens):
+// Whether the 16-token kernel takes a matrix (wide_ok) for mt pseudo-tokens in kernel mode 0: by the tokens alone, so
+// that a matrix gives the same bits in a group and on its own. For 2..4 fp16 tokens k_fused_tiles_mma stays: us per call
+// against this kernel, Q4_K gate + up 29.3 / 29.5 at 2 tokens, 31.0 / 29.4 at 4, 31.6 / 29.2 at 5, 36.2 / 29.4 at 8, a
+// whole layer 43.5 / 46, 47.5 / 46, 52.5 / 46.3, 59.6 / 47; Q5_K gate + up 38.2 / 44.2 at 2, 44.0 / 44.2 at 5 (its waves
+// take tile after tile, so many tiles per CU cost it one start; with few per CU this kernel is ahead at 2 as well).
+bool wide_takes(int mt, int per) { return g_kernel_mode == 0 && mt <= 16 && (per == 2 ? mt >= 2 : mt >= 5); }
+
+// Its blocks (a wave per half tile; sets the entries' w and block0 and the plan's W): rows of at most 8 units whole, so
+// that a row's sum stays in the block (us per call at 5 tokens, rows of 8: q, k and v 13.3 with 8 waves, 15.0 with 4),
+// longer ones 4 units at a time, small blocks that follow each other out of step (rows of 16 and 56, Q5_K: gate + up 44.2
+// / 49.1 / 59.2 with 4 / 8 / 16, down 29.9 / 31.8 / 36.2). Every block 4 units where a CU runs many blocks one after the
+// other (a whole Q4_K layer 46.3, with 8 48.3) or the units lie in long rows mostly, or 8 buffers do not fit the LDS.
+void wide_blocking(lw::WidePlan& wp) {
+  long long units = 0, rows = 0;
+  for (int i = 0; i < wp.n; ++i) {
+    const long long u = 2ll * wp.e[i].M.NT * wp.e[i].M.KT;
+    units += u;
+    if (wp.e[i].M.KT <= 8) rows += u;
+  }
+  const int rows_w = 2 * rows >= units && units <= 40ll * cu_count() &&
+                             lw::wide_lds_bytes(8, lw::wide_buf_rows(wp)) <= 160 * 1024
+                         ? 8
+                         : 4;
+  int blocks = 0;
+  wp.W = 1;
+  for (int i = 0; i < wp.n; ++i) {
+    lw::WideEntry& e = wp.e[i];
+    e.w = e.M.KT <= 8 ? rows_w : 4;
+    e.block0 = blocks;
+    blocks += lw::wide_blocks(e.M, e.w);
+    wp.W = std::max(wp.W, e.M.KT <= e.w ? e.w / e.M.KT * e.M.KT : e.w);
+  }
+}
+
+// Fused GEMV / skinny GEMM of `count` matrices with fp16 activations X[i] ([m * per][K_i] pseudo-tokens; x_f32, one
+// matrix, per = 2: fp32 [m][K], split into fp16 hi + lo on the device; twin: by the kernels that give a packed twin the
+// same bits):
 // ring-capable matrices go into grouped launches (same K-quant type and ring size, up to MAX_GROUP per launch), the
 // others into whole-tile launches. The ordered reduction over tile columns runs inside the flat (m = 1) launch for
 // every matrix that launch decodes completely, else in one reduction launch per MAX_GROUP matrices. Partials of
 // all matrices live side by side in the model's P scratch; calls that overlap on one model race (P and counters).
 // `launches` (optional) counts the kernel launches. x8 (flat kernels only; m = 1, or up to 8 tokens in one pass with
 // kernel modes 0, 3-5 and no packed matrix): int8 activations (quant_x8_dev) instead of X16.
-int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int count, int m, int per, float* const* Y,
+int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X, int count, int m, int per, float* const* Y,
                     const int* ldy, hipStream_t s, int* launches = nullptr, const X8* x8 = nullptr,
-                    const FixedScratch* fixed = nullptr) {
+                    const FixedScratch* fixed = nullptr, bool x_f32 = false, bool twin = false) {
   const int mt = m * per;
   std::vector<size_t> off(count + 1, 0);
   for (int i = 0; i < count; ++i) off[i + 1] = off[i] + (size_t)ts[i]->dm.KT * mt * ts[i]->N;
@@ -672,12 +713,13 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int cou
   // partials and counters: the model's (grown on demand) or a caller's fixed scratch (nothing allocated; its counters
   // and partial slots are set by fill kernels on the stream, since the last call on that scratch may have left
   // anything there). Partial slots hold kNoPartial outside a reduction (lw_kernels.h).
-  // 2..8 tokens of fp16 activations, every format: the whole-tile kernel with its products on the matrix cores
+  // 2..4 tokens of fp16 activations, every format: the whole-tile kernel with its products on the matrix cores
   auto mma_ok = [&](const lw::DevMat& dm) {
     return dm.kqt >= lw::KQ_Q4_K && dm.kqt <= lw::KQ_IQ4_XS && !dm.packed && dm.dsplit && dm.lut4 && dm.rows &&
            dm.max_rows + 2 <= 256;
   };
-  const bool mma = !x8 && per == 1 && mt >= 2 && mt <= 8 && g_kernel_mode == 0;
+  const bool wide = !x8 && !twin && wide_takes(mt, per);
+  const bool mma = !x8 && per == 1 && mt >= 2 && mt <= 4 && g_kernel_mode == 0;
   // its launches: matrices of one K-quant type, or of two (entries of the smaller type code first: one launch fewer),
   // up to MAX_GROUP each
   struct MmaLaunch {
@@ -708,7 +750,7 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int cou
           if (!pass) ++L.fp.nfa;
           lw::FlatEntry& e = L.fp.e[L.fp.n++];
           e.M = dm;
-          e.X2 = static_cast<const uint32_t*>(X16[j]);
+          e.X2 = static_cast<const uint32_t*>(X[j]);
           e.tile0 = L.fp.ntiles;
           e.ntile = dm.NT * dm.KT;
           e.Y = Y[j];
@@ -733,7 +775,7 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int cou
         if (mdone[j] || !mma_ok(dm) || dm.kqt != ts[i]->dm.kqt) continue;
         lw::FlatEntry& e = L.fp.e[L.fp.n++];
         e.M = dm;
-        e.X2 = static_cast<const uint32_t*>(X16[j]);
+        e.X2 = static_cast<const uint32_t*>(X[j]);
         e.tile0 = L.fp.ntiles;
         e.ntile = dm.NT * dm.KT;
         e.Y = Y[j];
@@ -750,10 +792,11 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int cou
   }
   float* Pb = nullptr;
   uint32_t* Cb = nullptr;
+  size_t fixed_need = 0;
   if (fixed) {
     const size_t cnt_bytes = (coff[count] * sizeof(uint32_t) + 255) & ~(size_t)255;
     const size_t p_bytes = (off[count] * sizeof(float) + 255) & ~(size_t)255;
-    const size_t need = cnt_bytes + p_bytes;
+    const size_t need = fixed_need = cnt_bytes + p_bytes;
     if (need > fixed->bytes) {
       g_err = "scratch of " + std::to_string(fixed->bytes) + " bytes is too small: this call needs " +
               std::to_string(need);
@@ -816,6 +859,70 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X16, int cou
   std::vector<lw::FlatPlan> flat_plans, split_plans;
   std::vector<std::pair<lw::FlatPlan, int>> tile_plans;  // whole-tile kernel launches and their tiles per block
   std::vector<std::pair<lw::FlatPlan, int>> half_plans;  // half-tile kernel launches and their tiles per block
+  // the 16-token whole-tile kernel over up to MAX_GROUP matrices of any formats, every tile and the reduction in the
+  // launch; the activations reordered first, each vector of the call once per symbol width
+  while (wide) {
+    lw::WidePlan wp{};
+    lw::WideXJobs xj{};
+    std::vector<int> sel, job;
+    size_t xbytes[lw::MAX_GROUP] = {}, xtotal = 0;
+    for (int j = 0; j < count && wp.n < lw::MAX_GROUP; ++j) {
+      const lw::DevMat& dm = ts[j]->dm;
+      if (done[j] || !lw::wide_ok(dm)) continue;
+      int k = 0;
+      while (k < xj.n && !(xj.X[k] == X[j] && xj.K[k] == dm.K && xj.symbits[k] == dm.symbits)) ++k;
+      if (k == xj.n) {
+        xj.X[k] = X[j];
+        xj.K[k] = dm.K;
+        xj.symbits[k] = dm.symbits;
+        xbytes[k] = xtotal;
+        xtotal += (lw::wide_x_bytes(mt, dm.K) + 255) & ~(size_t)255;
+        ++xj.n;
+      }
+      lw::WideEntry& e = wp.e[wp.n++];
+      e.M = dm;
+      job.push_back(k);
+      e.P = Pb + off[j];
+      e.Y = Y[j];
+      e.cnt = Cb + coff[j];
+      e.ldy = ldy[j];
+      sel.push_back(j);
+    }
+    if (!wp.n) break;
+    wp.mt = xj.mt = mt;
+    wp.per = per;
+    wide_blocking(wp);
+    xj.per = x_f32 ? 2 : 1;
+    uint8_t* xt;
+    if (fixed) {  // (one matrix) after the call's partials, or in their tail: a row has a slot per block, not per tile
+      const lw::DevMat& dm = wp.e[0].M;
+      const size_t slots = (size_t)((dm.KT + wp.e[0].w - 1) / wp.e[0].w) * m * dm.N;
+      const size_t used = (size_t)(reinterpret_cast<uint8_t*>(Pb) - fixed->base) + ((slots * sizeof(float) + 255) & ~(size_t)255);
+      const size_t at = fixed_need + xtotal <= fixed->bytes ? fixed_need : used;
+      if (count != 1 || at + xtotal > fixed->bytes) break;
+      xt = fixed->base + at;
+    } else {
+      if (grow(M.XW, M.XW_cap, xtotal)) return -1;
+      xt = M.XW;
+    }
+    for (int k = 0; k < wp.n; ++k) wp.e[k].X = xj.XT[job[k]] = xt + xbytes[job[k]];
+    for (int j : sel) done[j] = reduced[j] = exc_in[j] = whole[j] = 1;
+    HIPCHECK(lw::launch_wide_x(xj, s));
+    HIPCHECK(lw::launch_fused_wide(wp, s));
+    if (launches) *launches += 2;
+  }
+  std::vector<const void*> xh(X, X + count);  // fp16 pseudo-tokens
+  if (x_f32 && !done[0]) {
+    uint16_t* x16 = fixed ? fixed->x16 : nullptr;
+    if (!fixed) {
+      if (grow(M.X16, M.X16_cap, (size_t)mt * ts[0]->K * 2)) return -1;
+      x16 = M.X16;
+    }
+    HIPCHECK(lw::launch_split_x(static_cast<const float*>(X[0]), x16, m, (int)ts[0]->K, s));
+    if (launches) ++*launches;
+    xh[0] = x16;
+  }
+  const void* const* const X16 = xh.data();
   // packed (fixed-rate) matrices: the decode-free kernels, one launch per K-quant type and MAX_GROUP matrices
   // (m = 1: the flat one, which also reduces)
   for (int i = 0; mt == 1 && i < count; ++i) {
@@ -1220,9 +1327,16 @@ int group_matmul(Model& M, Tensor* const* ts, const void* const* X, int count, i
   return fused_group_dev(M, ts, X, count, m, 1, Y, ldy, s, launches);
 }
 
-int fused_dev(Model& M, Tensor& t, const void* X16, int m, int per, float* Y, int ldy, hipStream_t s) {
+int fused_dev(Model& M, Tensor& t, const void* X16, int m, float* Y, int ldy, hipStream_t s) {
   Tensor* tp = &t;
-  return fused_group_dev(M, &tp, &X16, 1, m, per, &Y, &ldy, s);
+  return fused_group_dev(M, &tp, &X16, 1, m, 1, &Y, &ldy, s);
+}
+
+// the same for fp32 activations on the device, m <= 8
+int fused_dev_f32(Model& M, Tensor& t, const void* X, int m, float* Y, int ldy, hipStream_t s,
+                  const FixedScratch* fixed = nullptr) {
+  Tensor* tp = &t;
+  return fused_group_dev(M, &tp, &X, 1, m, 2, &Y, &ldy, s, nullptr, nullptr, fixed, true);
 }
 
 // Prefill GEMM of path 2: 0 (default) = the hand-written MFMA GEMM over tiled codes for every K-quant format
@@ -1514,7 +1628,10 @@ int rt_test_matmul(void* h, const char* name, const float* X, int m, float* Y, i
       g_err = "rt_test_matmul: upload failed";
       return -1;
     }
-    rc = fused_dev(*M, *t, dx16, m, 2, dy, (int)N, M->stream);
+    // (the entry compares a matrix with its packed twin: the kernels that give both the same bits)
+    const void* xp = dx16;
+    const int ld = (int)N;
+    rc = fused_group_dev(*M, &t, &xp, 1, m, 2, &dy, &ld, M->stream, nullptr, nullptr, nullptr, false, true);
   } else {
     if (hipMalloc(reinterpret_cast<void**>(&dx), (size_t)m * K * 4) != hipSuccess ||
         hipMemcpy(dx, X, (size_t)m * K * 4, hipMemcpyHostToDevice) != hipSuccess) {
@@ -1741,16 +1858,14 @@ int lw_matmul_dev(void* h, const char* name, const void* X, int x_f16, int m, fl
       g_err = "lw_matmul_dev: fp16 activations need 1 <= m <= 16";
       return -1;
     }
-    return fused_dev(*M, *t, X, m, 1, Y, ldy, s);
+    return fused_dev(*M, *t, X, m, Y, ldy, s);
   }
   if (m < 1) {
     g_err = "lw_matmul_dev: m < 1";
     return -1;
   }
   if (m > 8) return decode_gemm_dev(*M, *t, static_cast<const float*>(X), m, Y, ldy, s);  // prefill shapes
-  if (grow(M->X16, M->X16_cap, (size_t)2 * m * t->K * 2)) return -1;
-  HIPCHECK(lw::launch_split_x(static_cast<const float*>(X), M->X16, m, (int)t->K, s));
-  return fused_dev(*M, *t, M->X16, m, 2, Y, ldy, s);
+  return fused_dev_f32(*M, *t, X, m, Y, ldy, s);
 }
 
 int lw_matmul_dev_noalloc(void* h, const char* name, const void* X, int x_f16, int m, float* Y, int ldy,
@@ -1774,9 +1889,8 @@ int lw_matmul_dev_noalloc(void* h, const char* name, const void* X, int x_f16, i
   if (!base) return -1;
   hipStream_t s = static_cast<hipStream_t>(stream);
   FixedScratch fx{base, kNoAllocScratchBytes};
-  const void* X16 = X;
-  int per = 1;
-  if (!x_f16) {  // fp32 x split into fp16 hi + lo rows, at the end of the scratch
+  int rc;
+  if (!x_f16) {  // fp32 x split into fp16 hi + lo, at the end of the scratch
     const size_t xb = ((size_t)2 * m * t->K * sizeof(uint16_t) + 255) & ~(size_t)255;
     if (xb >= fx.bytes) {
       g_err = "lw_matmul_dev_noalloc: activations exceed the " + std::to_string(kNoAllocScratchBytes) +
@@ -1784,12 +1898,11 @@ int lw_matmul_dev_noalloc(void* h, const char* name, const void* X, int x_f16, i
       return -1;
     }
     fx.bytes -= xb;
-    void* x16 = base + fx.bytes;
-    HIPCHECK(lw::launch_split_x(static_cast<const float*>(X), x16, m, (int)t->K, s));
-    X16 = x16;
-    per = 2;
+    fx.x16 = reinterpret_cast<uint16_t*>(base + fx.bytes);
+    rc = fused_dev_f32(*M, *t, X, m, Y, ldy, s, &fx);
+  } else {
+    rc = fused_group_dev(*M, &t, &X, 1, m, 1, &Y, &ldy, s, nullptr, nullptr, &fx);
   }
-  const int rc = fused_group_dev(*M, &t, &X16, 1, m, per, &Y, &ldy, s, nullptr, nullptr, &fx);
   if (rc) g_err = "lw_matmul_dev_noalloc: " + g_err;
   return rc;
 }

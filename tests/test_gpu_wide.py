@@ -1,0 +1,114 @@
+"""The 16-token half-tile kernel (lw_wide.hip) through the C-ABI, against fp64: every format, the smallest shapes and the
+ones that put a row of units into one block, across two and across many, 5..16 tokens of fp16 and 1..8 of fp32
+activations, groups of several formats in one call, activations at any alignment, and a caller's scratch at its limit."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# fp32 sums of exact products, K <= 28672 terms in sums of 16: 2-norm errors of a few 2^-24
+TOL = 1e-6
+H = {1: 2.3, 2: 3.4, 3: 4.3, 4: 2.6}
+
+
+def open_mats(tmp_path, mats):
+    from lazyweights_amd import Runtime, bundle
+    bundle.write_synthetic_bundle(str(tmp_path), mats, threads=16)
+    rt = Runtime(tmp_path)
+    w = {}
+    for name, kqt, N, K, h, seed in mats:
+        w[name] = bundle.synth_matrix(kqt, N, K, h, seed, threads=16)
+    return rt, w
+
+
+def y64(orc, kqt, w, x):
+    return orc.gemv_f64(orc.dequant(kqt, *w), x.float().cpu().double().numpy())
+
+
+def err(y, ref):
+    y = y.double().cpu().numpy()
+    return np.linalg.norm(y - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("kqt", (1, 2, 3, 4))
+def test_formats_shapes_and_tokens(gpu, lib, orc, tmp_path, kqt):
+    import torch
+    cols = 512 if kqt in (1, 4) else 256
+    # units per row: 1, 3, 8 (a block holds whole rows), 9 (4-wave blocks, rows shared), 28 in a tall matrix
+    mats = [("r%d" % i, kqt, n, k * cols, H[kqt], 900 + i)
+            for i, (n, k) in enumerate(((64, 1), (192, 3), (320, 8), (128, 9), (640, 28)))]
+    rt, w = open_mats(tmp_path, mats)
+    try:
+        for name, _, N, K, _, seed in mats:
+            for m, f16 in ((5, True), (7, True), (9, True), (16, True), (1, False), (3, False), (8, False)):
+                g = torch.Generator().manual_seed(seed + m)
+                x = torch.randn(m, K, generator=g)
+                x = (x.half() if f16 else x).cuda()
+                y = torch.full((m, N + 3), float("nan"), device="cuda")
+                for _ in range(2):  # the second call finds slots and counters as the first left them
+                    assert lib.lw_matmul_dev(rt.h, name.encode(), x.data_ptr(), int(f16), m, y.data_ptr(), N + 3, None) == 0
+                torch.cuda.synchronize()
+                e = err(y[:, :N], y64(orc, kqt, w[name], x))
+                print(name, kqt, N, K, m, f16, "err %.2g" % e, flush=True)
+                assert e < TOL
+                assert torch.isnan(y[:, N:]).all()
+    finally:
+        rt.close()
+
+
+def test_group_of_formats_and_alignment(gpu, lib, orc, tmp_path):
+    import torch
+    mats = [("a", 1, 256, 4096, H[1], 1), ("b", 3, 128, 4096, H[3], 2), ("c", 2, 192, 1024, H[2], 3),
+            ("d", 4, 64, 4096, H[4], 4)] + [("e%d" % i, 1 + i % 4, 64, 1024, H[1 + i % 4], 5 + i) for i in range(6)]
+    rt, w = open_mats(tmp_path, mats)
+    try:
+        for m, shift in ((6, 0), (16, 1), (7, 4)):  # x shared by equal K, `shift` fp16 past a 16-byte boundary
+            xs = {}
+            for K in (1024, 4096):
+                buf = torch.zeros(m * K + 8, dtype=torch.float16, device="cuda")
+                buf[shift:shift + m * K] = torch.randn(m * K, generator=torch.Generator().manual_seed(m + K)).half().cuda()
+                xs[K] = buf[shift:shift + m * K].view(m, K)
+            ys = [torch.zeros(m, mat[2], device="cuda") for mat in mats]
+            n = len(mats)
+            assert lib.lw_group_matmul_dev(rt.h, n, (ctypes.c_char_p * n)(*[mt[0].encode() for mt in mats]),
+                                           (ctypes.c_void_p * n)(*[xs[mt[3]].data_ptr() for mt in mats]), m,
+                                           (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys]), None) == 0
+            torch.cuda.synchronize()
+            for mt, y in zip(mats, ys):
+                assert err(y, y64(orc, mt[1], w[mt[0]], xs[mt[3]])) < TOL, (mt, m, shift)
+    finally:
+        rt.close()
+
+
+def test_token_order_nan_and_scratch_limit(gpu, lib, orc, tmp_path):
+    """A NaN token leaves the others their bits and the partial slots consistent; without allocation the reordered
+    activations go into the partials' tail where the 16 MiB hold no more (16 x 8 x 32768 partials are exactly that less
+    the counters, so 32256 rows are the most)."""
+    import torch
+    mats = [("m", 1, 32256, 4096, 2.3, 11), ("s", 1, 128, 4608, 2.3, 12)]
+    rt, w = open_mats(tmp_path, mats)
+    try:
+        K = 4096
+        x = torch.randn(16, K, generator=torch.Generator().manual_seed(3)).half().cuda()
+        ya, yb = (torch.zeros(16, 32256, device="cuda") for _ in range(2))
+        for fn, y in ((lib.lw_matmul_dev, ya), (lib.lw_matmul_dev_noalloc, yb)):
+            assert fn(rt.h, b"m", x.data_ptr(), 1, 16, y.data_ptr(), 32256, None) == 0, lib.lw_last_error()
+        torch.cuda.synchronize()
+        assert torch.equal(ya, yb)
+        assert err(ya, y64(orc, 1, w["m"], x)) < TOL
+        x = torch.randn(9, 4608, generator=torch.Generator().manual_seed(4)).half().cuda()
+        ref, y = (torch.zeros(9, 128, device="cuda") for _ in range(2))
+        lib.lw_matmul_dev(rt.h, b"s", x.data_ptr(), 1, 9, ref.data_ptr(), 128, None)
+        bad = x.clone()
+        bad[4, 100] = float("nan")
+        lib.lw_matmul_dev(rt.h, b"s", bad.data_ptr(), 1, 9, y.data_ptr(), 128, None)
+        torch.cuda.synchronize()
+        keep = [i for i in range(9) if i != 4]
+        assert torch.isnan(y[4]).all() and torch.equal(y[keep], ref[keep])
+        lib.lw_matmul_dev(rt.h, b"s", x.data_ptr(), 1, 9, y.data_ptr(), 128, None)
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+    finally:
+        rt.close()
