@@ -31,6 +31,7 @@ HIP_DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang",
 SOURCES = [
     ("lw_kernels.hip", "hip"),
     ("lw_wide.hip", "hip"),
+    ("lw_prefill.hip", "hip"),
     ("lw_runtime.cpp", "hiphost"),
     ("lw_codec.cpp", "cxx"),
     ("lw_layout.cpp", "cxx"),

@@ -241,18 +241,26 @@ hipError_t launch_dequant_hilo(const DevMat& M, const uint8_t* codes, int row0, 
 hipError_t launch_decode_hilo(const DevMat& M, int tr0, int tr1, void* WW, hipStream_t s);
 // Prefill GEMM on the matrix cores, every K-quant format (k_gemm_prefill: Q4_K / Q5_K; k_gemm_prefill_sub: Q6_K /
 // IQ4_XS): Y[t][row0 + r] for the chunk's rows r < nrows (a multiple of 64) from its codes in the tiled layout
-// (launch_decode_tiled) and x in the tiled layouts of launch_prefill_x (SXT read for Q4_K / Q5_K only); K a multiple
+// (launch_prefill_prep) and x in its tiled layouts (SXT read for Q4_K / Q5_K only); K a multiple
 // of 256
 hipError_t launch_gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int nrows, const void* XT,
                                const void* SXT, int m, float* Y, int ldy, hipStream_t s);
-// codes of tile rows [tr0, tr1) in the prefill GEMM's tiled layout: per 32-row tile and 32-code chunk a 1 KB piece,
+// Codes of tile rows [tr0, tr1) in the prefill GEMM's tiled layout: per 32-row tile and 32-code chunk a 1 KB piece,
 // lane (h, c) = 32 h + c holding row c's codes 16 h .. 16 h + 15 of the chunk (IQ4_XS: their grid bytes kv[q] + 128);
-// hipErrorNotSupported unless decode_tiled_ok (packed matrices, coded ones with split offsets)
+// needs decode_tiled_ok (packed matrices, coded ones with split offsets). With x in the same launch: fp32 X [m][K] -> XT
+// (fp16 hi / lo pieces, prefill_x_bytes) and SXT (per-sub-block sums as fp16 hi / lo, prefill_sx_bytes; null: none),
+// tokens padded with zeros to a multiple of 64; K a multiple of 256.
+struct PrefillX {
+  const float* X;
+  uint16_t* XT;
+  uint16_t* SXT;
+  int m, K;
+  int blocks;  // set by the launch
+};
 bool decode_tiled_ok(const DevMat& M);
-hipError_t launch_decode_tiled(const DevMat& M, uint8_t* out, int tr0, int tr1, hipStream_t s);
-// fp32 X [m][K] -> XT (fp16 hi / lo pieces, prefill_x_bytes) and SXT (per-sub-block sums as fp16 hi / lo,
-// prefill_sx_bytes), tokens padded with zeros to a multiple of 64; K a multiple of 256
-hipError_t launch_prefill_x(const float* X, void* XT, void* SXT, int m, int K, hipStream_t s);
+hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, const PrefillX* x, hipStream_t s);
+// the codes of a packed matrix in that layout
+hipError_t launch_unpack_tiled(const DevMat& M, uint8_t* out, int tr0, int tr1, hipStream_t s);
 size_t prefill_x_bytes(int m, int K);
 size_t prefill_sx_bytes(int m, int K);
 // x [m][K] fp32 -> XB [2m][2K] fp16: rows t < m [hi | hi], rows m + t [lo | 0]
