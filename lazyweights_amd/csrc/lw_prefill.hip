@@ -188,10 +188,16 @@ hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, 
 // Operand layout (32x32x16): lane l holds A[i = l % 32][k = 8 (l / 32) + 0..7] (token i) and B[k = 8 (l / 32) + 0..7]
 // [j = l % 32] (weight row j), and receives D[i = 8 (r / 4) + 4 (l / 32) + r % 4][j = l % 32] in register r: a lane owns
 // one weight row (one set of scales) per row tile and 16 tokens of the token tile.
-// Block = GEMM_WAVES waves over 64 weight rows (two row tiles) x 32 tokens; the waves split K by super-block (wave w
-// takes super-blocks w, w + GEMM_WAVES, ...) and their partial tiles are summed through LDS in wave order, so the
-// result does not depend on timing. A skinny prefill (m = 128, N = 4096) gives 256 blocks.
-constexpr int GEMM_WAVES = 8;
+// Block = WV waves over 64 weight rows (two row tiles) x 32 TT tokens; the waves split K by super-block (wave w takes
+// super-blocks w, w + WV, ...) and their partial tiles are summed through LDS in wave order, so the result does not
+// depend on timing.
+// What bounds it: a wave of TT = 1 reads 6 KB of operands per 8 products (256 cycles of a SIMD's matrix core), 96 bytes a
+// cycle of a CU where its vector cache gives 64; with TT = 2 the same codes serve 16 products (80 bytes a cycle, and half
+// the scaling of codes per product). 64 x 64 tiles take all 256 registers of 2 waves per SIMD (128 in accumulators): the
+// operand rings are 2 chunks deep instead of 4, side records and x sums are read through buffers (no per-lane addresses)
+// half a super-block ahead, and a tile's registers take its mins product once it is folded. Q4_K 14336 x 4096, m = 2048:
+// 728 -> 516 us with the preparation, 496 useful TFLOP/s in the GEMM = 992 of products, where a library fp16 GEMM of
+// 8192 x 8192 x 8192 reaches 1176 on this card.
 // codes q0..q3 (bytes of qw) -> sc q / 16 as 4 fp16 in two words (nsc = -64 sc)
 __device__ __forceinline__ uint2 scaled_codes16(uint32_t qw, h2v sc, h2v nsc) {
   const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x54545454u, qw, 0x04010400u));
@@ -220,7 +226,7 @@ __device__ __forceinline__ h2v kside_sc(const KSide& k, int j) {
   const _Float16 v = (_Float16)(float)((((j < 4) ? k.sc_lo : k.sc_hi) >> (8 * (j & 3))) & 255u);
   return h2v{v, v};
 }
-// the 8 mins as the B operand of the mins product (k 0..7; lanes h = 1 pass zeros)
+// the 8 mins as the B operand of the mins product
 __device__ __forceinline__ h8v kside_mins(const KSide& k) {
   h8v v;
 #pragma unroll
@@ -239,71 +245,148 @@ __device__ __forceinline__ h8v kside_mins(const KSide& k) {
 //   SXT: per token tile tt, super-block sb and half a 512-byte piece, lane c (< 32) holding Sx[token c][8 sb + 0..7].
 // Step s of chunk kc gives lane (h, c) the weights 32 kc + 16 h + 8 s + 0..7 in both operands: the products of the
 // 32 weights of the chunk are all taken once, in a different order than k, which a dot product does not see.
+// The side records of one row of a wave's 64 through a buffer (no per-lane addresses): as the words side_load gives, but
+// Q6_K's 18 bytes as the 5 aligned dwords that hold them (side_words; a side tensor ends with 16 bytes of padding).
 template <int KQ>
-__global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill(DevMat M, const uint8_t* __restrict__ CT, int row0,
-                                                               const uint16_t* __restrict__ XT,
-                                                               const uint16_t* __restrict__ SXT, int m,
-                                                               float* __restrict__ Y, int ldy) {
+__device__ __forceinline__ uint32_t side_voffset(int c) { return (uint32_t)(c * kq_sbytes(KQ)) & (KQ == KQ_Q6_K ? ~3u : ~0u); }
+template <int KQ>
+__device__ __forceinline__ void side_fetch(__amdgpu_buffer_rsrc_t r, uint32_t vo, int so, uint32_t* w) {
+  if constexpr (KQ == KQ_IQ4_XS) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, vo, so, 0);
+    w[0] = v[0];
+    w[1] = v[1];
+  } else {
+    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = v[i];
+    if constexpr (KQ == KQ_Q6_K) w[4] = __builtin_amdgcn_raw_buffer_load_b32(r, vo + 16, so, 0);
+  }
+}
+template <int KQ>
+__device__ __forceinline__ void side_words(const uint32_t* raw, int c, uint32_t* w) {
+  const uint32_t sh = KQ == KQ_Q6_K ? 16u * (c & 1) : 0u;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = KQ == KQ_Q6_K ? __builtin_amdgcn_alignbit(raw[i + 1], raw[i], sh) : raw[i];
+  w[4] = KQ == KQ_Q6_K ? raw[4] >> sh : 0u;
+}
+
+// The block's pair of row tiles and first token tile. With TT = 2 (many blocks) in an order by XCD: hardware deals
+// consecutive blocks to the 8 XCDs, so block id takes place (id % 8) n / 8 + id / 8 of a list that runs over groups of 4
+// token tile pairs and inside a group over row pairs: an XCD's L2 keeps a group's activations while each row pair's codes
+// come by once (Q4_K 14336 x 4096, m = 2048: 528 -> 516 us, m = 512: 147 -> 143; groups of 1, 2 and 8: 529, 515, 529).
+template <int TT>
+__device__ __forceinline__ void block_tile(int& rp, int& tt) {
+  rp = blockIdx.x;
+  tt = blockIdx.y;
+  if constexpr (TT > 1) {
+    constexpr int G = 4;
+    const int gx = gridDim.x, gy = gridDim.y, per = gx * gy / 8;
+    int id = tt * gx + rp;
+    if (id < 8 * per) id = (id & 7) * per + (id >> 3);
+    const int g = id / (gx * G), rem = id - g * gx * G, gw = min(G, gy - g * G);
+    rp = rem / gw;
+    tt = g * G + rem - rp * gw;
+  }
+  tt *= TT;
+}
+
+// TT: token tiles of 32 per wave; WV: waves per block (the K split). The block's partial tiles -> LDS as
+// part[wave][tile][r][lane] (lane-contiguous, no bank conflicts), then each thread sums its outputs over the waves in
+// order; consecutive threads take consecutive lanes = consecutive weight rows. Tile = row tile + 2 token tile.
+template <int TT, int WV>
+__device__ __forceinline__ void store_tiles(const f16x16 (&tot)[2][TT], float* part, int wave, int lane, int row0, int tt0,
+                                            int m, float* __restrict__ Y, int ldy) {
+  constexpr int TILES = 2 * TT;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[((wave * TILES + a + 2 * b) * 16 + r) * 64 + lane] = tot[a][b][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < TILES * 16 * 64; e += 64 * WV) {
+    const int tile = e >> 10, r = (e >> 6) & 15, l = e & 63;
+    float acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < WV; ++w) acc += part[w * TILES * 1024 + e];
+    const int t = tt0 * 32 + 32 * (tile >> 1) + 8 * (r / 4) + 4 * (l >> 5) + (r % 4);
+    if (t < m) Y[(size_t)t * ldy + row0 + 32 * (tile & 1) + (l & 31)] = acc;
+  }
+}
+
+template <int KQ, int TT, int WV>
+__global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, const uint8_t* __restrict__ CT, int row0,
+                                                                     const uint16_t* __restrict__ XT,
+                                                                     const uint16_t* __restrict__ SXT, int m,
+                                                                     float* __restrict__ Y, int ldy) {
   static_assert(KQ == KQ_Q4_K || KQ == KQ_Q5_K, "scaled weights are exact in fp16 for Q4_K / Q5_K only");
   constexpr int SB = kq_sbytes(KQ), NSB = kq_symbits(KQ) == 4 ? 2 : 1;
+  constexpr int RD = TT == 1 ? 4 : 2;  // chunks on the operand rings (RD - 1 ahead)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  const int rp = blockIdx.x, tt = blockIdx.y;            // pair of 32-row tiles of the chunk, 32-token tile
+  const int lane = threadIdx.x & 63, c = lane & 31;
+  int rp, tt;  // pair of 32-row tiles of the chunk, first 32-token tile
+  block_tile<TT>(rp, tt);
   const int K = M.K, KC = K / 32, NB = K / 256;
-  const int nA = rp * 64 + c, nB = nA + 32;              // the lane's weight rows within the chunk
-  // buffer resources over the block's codes (its two row tiles) and x (its token tile): the lane's byte offset is
+  // buffer resources over the block's codes (its two row tiles) and x (its token tiles): the lane's byte offset is
   // the only per-lane address, the chunk offset a scalar
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(CT + (size_t)rp * 2 * KC * 1024), (short)0, 2 * KC * 1024, kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(XT + (size_t)tt * KC * 2048), (short)0, KC * 4096, kBufferRsrcWord3);
-  const uint16_t* sxw = SXT + (size_t)tt * NB * 512 + c * 8;
+      const_cast<uint16_t*>(XT + (size_t)tt * KC * 2048), (short)0, TT * KC * 4096, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(M.side + side_record(row0 + rp * 64, 0, M.KT, NSB) * SB), (short)0, NB * 64 * SB + 16, kBufferRsrcWord3);
+  const uint32_t vs = side_voffset<KQ>(c);  // row c's record, row c + 32's 32 SB on (a super-block's 64 records in a run)
+  const __amdgpu_buffer_rsrc_t rsx = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(SXT + (size_t)tt * NB * 512), (short)0, TT * NB * 1024, kBufferRsrcWord3);
   const uint32_t vo = (uint32_t)lane * 16;
-  // operands in flight: codes and x three chunks ahead on 4-slot rings (one depth for both: the load counter
-  // completes in issue order); 8 chunks per super-block keep the rings aligned
+  // operands in flight: codes and x RD - 1 chunks ahead (one depth for both: the load counter completes in issue order);
+  // 8 chunks per super-block keep the rings aligned
   auto load_q = [&](int kc, u32x4& qa, u32x4& qb) {
     qa = __builtin_amdgcn_raw_buffer_load_b128(rc, vo, kc * 1024, 0);
     qb = __builtin_amdgcn_raw_buffer_load_b128(rc, vo, (KC + kc) * 1024, 0);
   };
   auto load_x = [&](int kc, u32x4* x) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, vo + i * 1024, kc * 4096, 0);
-  };
-  f16x16 totA = {}, totB = {};
-  uint32_t swa[5] = {}, swb[5] = {};
-  u32x4 qa[4] = {}, qb[4] = {}, xr[4][4] = {};
-  if (wave < NB) {
-    side_load<KQ>(M.side + side_record(row0 + nA, wave, M.KT, NSB) * SB, swa);
-    side_load<KQ>(M.side + side_record(row0 + nB, wave, M.KT, NSB) * SB, swb);
+    for (int b = 0; b < TT; ++b)
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+      for (int i = 0; i < 4; ++i)
+        x[4 * b + i] = __builtin_amdgcn_raw_buffer_load_b128(rx, vo + i * 1024, (b * KC + kc) * 4096, 0);
+  };
+  f16x16 tot[2][TT] = {};
+  uint32_t swa[5] = {}, swb[5] = {};
+  u32x4 qa[RD] = {}, qb[RD] = {}, xr[RD][4 * TT] = {};
+  if (wave < NB) {
+    side_fetch<KQ>(rs, vs, wave * (64 * SB), swa);
+    side_fetch<KQ>(rs, vs + 32 * SB, wave * (64 * SB), swb);
+#pragma unroll
+    for (int i = 0; i < RD - 1; ++i) {
       load_q(wave * 8 + i, qa[i], qb[i]);
       load_x(wave * 8 + i, xr[i]);
     }
   }
-  for (int sb = wave; sb < NB; sb += GEMM_WAVES) {
+  for (int sb = wave; sb < NB; sb += WV) {
     const KSide ka = kside(swa), kb = kside(swb);
-    const int nsb = sb + GEMM_WAVES;
-    if (nsb < NB) {
-      side_load<KQ>(M.side + side_record(row0 + nA, nsb, M.KT, NSB) * SB, swa);
-      side_load<KQ>(M.side + side_record(row0 + nB, nsb, M.KT, NSB) * SB, swb);
-    }
-    uint4 sxh = {}, sxl = {};  // Sx of this super-block, loaded at chunk 5
-    f16x16 dA = {}, dB = {};
+    const int nsb = sb + WV;
+    u32x4 sx[TT];  // Sx of this super-block, loaded at chunk 5: lanes h = 0 the hi, h = 1 the lo halves
+    f16x16 d[2][TT] = {};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {  // the super-block's 8 chunks (sub-blocks)
-      if (j < 5 || nsb < NB) {
-        const int kn = j < 5 ? sb * 8 + j + 3 : nsb * 8 + j - 5;
-        load_q(kn, qa[(j + 3) & 3], qb[(j + 3) & 3]);
-        load_x(kn, xr[(j + 3) & 3]);
+      if (j < 9 - RD || nsb < NB) {
+        const int kn = j < 9 - RD ? sb * 8 + j + RD - 1 : nsb * 8 + j - (9 - RD);
+        load_q(kn, qa[(j + RD - 1) % RD], qb[(j + RD - 1) % RD]);
+        load_x(kn, xr[(j + RD - 1) % RD]);
       }
-      if (j == 5 && h == 0) {  // lanes h = 0 hold the mins product's k 0..7; k 8..15 stay zero
-        sxh = *reinterpret_cast<const uint4*>(sxw + (size_t)sb * 512);
-        sxl = *reinterpret_cast<const uint4*>(sxw + (size_t)sb * 512 + 256);
+      if (j == 5) {
+#pragma unroll
+        for (int b = 0; b < TT; ++b) sx[b] = __builtin_amdgcn_raw_buffer_load_b128(rsx, vo, (b * NB + sb) * 1024, 0);
+      }
+      if (j == 5 && nsb < NB) {  // the next super-block's records (from the start they would cost 10 registers more)
+        side_fetch<KQ>(rs, vs, nsb * (64 * SB), swa);
+        side_fetch<KQ>(rs, vs + 32 * SB, nsb * (64 * SB), swb);
       }
       __builtin_amdgcn_sched_barrier(0);  // keep the loads issued here, ahead of this chunk's products
-      const u32x4 ca = qa[j & 3], cb = qb[j & 3];
-      const u32x4* xc = xr[j & 3];
+      const u32x4 ca = qa[j % RD], cb = qb[j % RD];
+      const u32x4* xc = xr[j % RD];
       const h2v sca = kside_sc(ka, j), scb = kside_sc(kb, j);
       const h2v n64 = {(_Float16)-64.f, (_Float16)-64.f};
       const h2v nsa = sca * n64, nsb2 = scb * n64;
@@ -311,49 +394,44 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill(DevMat M, cons
       for (int st = 0; st < 2; ++st) {
         const uint2 a0 = scaled_codes16(ca[2 * st], sca, nsa), a1 = scaled_codes16(ca[2 * st + 1], sca, nsa);
         const uint2 b0 = scaled_codes16(cb[2 * st], scb, nsb2), b1 = scaled_codes16(cb[2 * st + 1], scb, nsb2);
-        const h8v wa = __builtin_bit_cast(h8v, make_uint4(a0.x, a0.y, a1.x, a1.y));
-        const h8v wb = __builtin_bit_cast(h8v, make_uint4(b0.x, b0.y, b1.x, b1.y));
-        const h8v xh = __builtin_bit_cast(h8v, xc[st]), xl = __builtin_bit_cast(h8v, xc[2 + st]);
-        dA = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, wa, dA, 0, 0, 0);
-        dB = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, wb, dB, 0, 0, 0);
-        dA = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, wa, dA, 0, 0, 0);
-        dB = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, wb, dB, 0, 0, 0);
+        const h8v w[2] = {__builtin_bit_cast(h8v, make_uint4(a0.x, a0.y, a1.x, a1.y)),
+                          __builtin_bit_cast(h8v, make_uint4(b0.x, b0.y, b1.x, b1.y))};
+#pragma unroll
+        for (int half = 0; half < 2; ++half)  // x hi, then lo
+#pragma unroll
+          for (int b = 0; b < TT; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+              d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, xc[4 * b + 2 * half + st]), w[a], d[a][b], 0, 0, 0);
       }
     }
-    // mins: A2 = the tokens' Sx over the super-block's 8 sub-blocks, B2 = the row's 8 mins
-    h8v ma = {}, mb = {};
-    if (h == 0) {
-      ma = kside_mins(ka);
-      mb = kside_mins(kb);
+    // mins: A2 = the tokens' Sx over the super-block's 8 sub-blocks, hi in k 0..7 and lo in k 8..15, B2 = the row's 8
+    // mins in both
+    const h8v mn[2] = {kside_mins(ka), kside_mins(kb)};
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const float d16 = a ? kb.d16 : ka.d16;
+#pragma unroll
+      for (int b = 0; b < TT; ++b) {
+        // (the tile's registers take the mins product once they are folded)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(d16, d[a][b][r], tot[a][b][r]);
+        asm volatile("" : "+v"(tot[a][b]));
+        d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sx[b]), mn[a], f16x16{}, 0, 0, 0);
+      }
     }
-    f16x16 mA = {}, mB = {};
-    mA = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sxh), ma, mA, 0, 0, 0);
-    mB = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sxh), mb, mB, 0, 0, 0);
-    mA = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sxl), ma, mA, 0, 0, 0);
-    mB = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sxl), mb, mB, 0, 0, 0);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      totA[r] = fmaf(ka.d16, dA[r], fmaf(-ka.dmin, mA[r], totA[r]));
-      totB[r] = fmaf(kb.d16, dB[r], fmaf(-kb.dmin, mB[r], totB[r]));
+    for (int a = 0; a < 2; ++a) {
+      const float dmin = a ? kb.dmin : ka.dmin;
+#pragma unroll
+      for (int b = 0; b < TT; ++b) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(-dmin, d[a][b][r], tot[a][b][r]);
+      }
     }
   }
-  // partial tiles -> LDS as part[wave][row tile][r][lane] (lane-contiguous, no bank conflicts), then each thread
-  // sums its outputs over the waves in order; consecutive threads take consecutive lanes = consecutive weight rows
-  __shared__ float part[GEMM_WAVES][2][16][64];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    part[wave][0][r][lane] = totA[r];
-    part[wave][1][r][lane] = totB[r];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 2 * 16 * 64; e += 64 * GEMM_WAVES) {
-    const int half = e >> 10, r = (e >> 6) & 15, l = e & 63;
-    float acc = 0.f;
-#pragma unroll
-    for (int w = 0; w < GEMM_WAVES; ++w) acc += part[w][half][r][l];
-    const int t = tt * 32 + 8 * (r / 4) + 4 * (l >> 5) + (r % 4);
-    if (t < m) Y[(size_t)t * ldy + row0 + rp * 64 + 32 * half + (l & 31)] = acc;
-  }
+  extern __shared__ float part[];
+  store_tiles<TT, WV>(tot, part, wave, lane, row0 + rp * 64, tt, m, Y, ldy);
 }
 
 // ── prefill GEMM on the matrix cores, Q6_K / IQ4_XS: unscaled grid weights, folded per sub-block ─────────────
@@ -361,15 +439,17 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill(DevMat M, cons
 // at most 8 bits, exact in fp16, where the scaled s f(q) (up to 128 x 32 or 32 x 127) is not. Each sub-block's
 // products go to a fresh accumulator tile (x split into fp16 hi + lo, as k_gemm_prefill), folded into the fp32 total
 // with d s_j (exact in fp32) once the sub-block is in. No offsets: neither format has mins.
-// The block, the waves' split of K, the rings and the wave-order LDS sum are those of k_gemm_prefill. A step's K = 16
+// The block, the waves' split of K, the rings and the wave-order LDS sum are those of k_gemm_prefill; the fold (an FMA per
+// output and sub-block) is as much VALU as there is matrix-core time for Q6_K: 4096 x 14336, m = 512 takes 170 us (64 x 32
+// tiles 200). A step's K = 16
 // must lie in one sub-block:
 //   IQ4_XS (32-weight sub-blocks) takes k_gemm_prefill's steps (a chunk = a sub-block) over the grid bytes kv[q] + 128
 //   of the tiled codes; weights fp16(1024 + g) from a byte permute against 0x64, minus 1152.
 //   Q6_K (16-weight sub-blocks) takes weights 16 s + 8 h + 0..7 of the chunk in step s for lane (h, c), so that step s
 //   is sub-block 2 kc + s: 8 bytes of the codes piece at lane slot 32 s + c, byte 8 h, and the x piece of step h at
 //   lane slot 32 s + c (the products of a chunk are still each taken once); weights fp16(1024 + q) minus 1056.
-template <int KQ>
-__global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill_sub(DevMat M, const uint8_t* __restrict__ CT, int row0,
+template <int KQ, int TT, int WV>
+__global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill_sub(DevMat M, const uint8_t* __restrict__ CT, int row0,
                                                                    const uint16_t* __restrict__ XT, int m,
                                                                    float* __restrict__ Y, int ldy) {
   static_assert(KQ == KQ_Q6_K || KQ == KQ_IQ4_XS, "per-sub-block folding: Q6_K and IQ4_XS");
@@ -377,13 +457,17 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill_sub(DevMat M, 
   constexpr int SB = kq_sbytes(KQ), NSB = kq_symbits(KQ) == 4 ? 2 : 1;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
-  const int rp = blockIdx.x, tt = blockIdx.y;
+  constexpr int RD = TT == 1 ? 4 : 2;  // chunks on the operand rings (RD - 1 ahead)
+  int rp, tt;
+  block_tile<TT>(rp, tt);
   const int K = M.K, KC = K / 32, NB = K / 256;
-  const int nA = rp * 64 + c, nB = nA + 32;
   const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(CT + (size_t)rp * 2 * KC * 1024), (short)0, 2 * KC * 1024, kBufferRsrcWord3);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint16_t*>(XT + (size_t)tt * KC * 2048), (short)0, KC * 4096, kBufferRsrcWord3);
+      const_cast<uint16_t*>(XT + (size_t)tt * KC * 2048), (short)0, TT * KC * 4096, kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(M.side + side_record(row0 + rp * 64, 0, M.KT, NSB) * SB), (short)0, NB * 64 * SB + 16, kBufferRsrcWord3);
+  const uint32_t vs = side_voffset<KQ>(c);  // row c's record, row c + 32's 32 SB on (a super-block's 64 records in a run)
   // the lane's byte offsets of step s's operands in a chunk's codes piece and in its x pieces (hi, then lo 2 KB on)
   uint32_t vq[2], vx[2];
 #pragma unroll
@@ -410,7 +494,10 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill_sub(DevMat M, 
   };
   auto load_x = [&](int kc, u32x4* x) {  // x[2 half + s]
 #pragma unroll
-    for (int i = 0; i < 4; ++i) x[i] = __builtin_amdgcn_raw_buffer_load_b128(rx, vx[i & 1] + (i >> 1) * 2048, kc * 4096, 0);
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        x[4 * b + i] = __builtin_amdgcn_raw_buffer_load_b128(rx, vx[i & 1] + (i >> 1) * 2048, (b * KC + kc) * 4096, 0);
   };
   // 4 weights (bytes of qw) -> fp16 f(q) in two words
   const h2v bias = Q6 ? h2v{(_Float16)-1056.f, (_Float16)-1056.f} : h2v{(_Float16)-1152.f, (_Float16)-1152.f};
@@ -425,101 +512,152 @@ __global__ void __launch_bounds__(64 * GEMM_WAVES) k_gemm_prefill_sub(DevMat M, 
     const uint32_t ls = ((w[1] >> (4 * j)) & 15u) | ((w[0] >> (16 + 2 * j)) & 3u) << 4;
     return h2f(w[0]) * (float)((int)ls - 32);
   };
-  f16x16 totA = {}, totB = {};
+  f16x16 tot[2][TT] = {};
+  extern __shared__ float part[];
+  // a total takes 8 or 16 rounded additions per super-block: half way (with 4 waves sharing K)
+  // it is put aside in the wave's part of the LDS, which keeps the sums' distance from 64 bits (Q6_K, K = 14336 and 4096:
+  // 2.1e-7 and 1.3e-7 with 8 waves and with this, 2.8e-7 and 1.6e-7 with 4 waves without it)
+  int left = WV < 8 ? ((NB - wave + WV - 1) / WV + 1) / 2 : 0;
+  bool aside = false;
+  f4v* const own = reinterpret_cast<f4v*>(part) + wave * 2 * TT * 256 + lane;  // [tile][r / 4][lane]
   uint32_t swa[5] = {}, swb[5] = {};
-  u32x4 qa[4] = {}, qb[4] = {}, xr[4][4] = {};
+  u32x4 qa[RD] = {}, qb[RD] = {}, xr[RD][4 * TT] = {};
   if (wave < NB) {
-    side_load<KQ>(M.side + side_record(row0 + nA, wave, M.KT, NSB) * SB, swa);
-    side_load<KQ>(M.side + side_record(row0 + nB, wave, M.KT, NSB) * SB, swb);
+    side_fetch<KQ>(rs, vs, wave * (64 * SB), swa);
+    side_fetch<KQ>(rs, vs + 32 * SB, wave * (64 * SB), swb);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
+    for (int i = 0; i < RD - 1; ++i) {
       load_q(wave * 8 + i, qa[i], qb[i]);
       load_x(wave * 8 + i, xr[i]);
     }
   }
-  for (int sb = wave; sb < NB; sb += GEMM_WAVES) {
-    uint32_t wa[5], wb[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      wa[i] = swa[i];
-      wb[i] = swb[i];
-    }
-    const int nsb = sb + GEMM_WAVES;
-    if (nsb < NB) {
-      side_load<KQ>(M.side + side_record(row0 + nA, nsb, M.KT, NSB) * SB, swa);
-      side_load<KQ>(M.side + side_record(row0 + nB, nsb, M.KT, NSB) * SB, swb);
-    }
+  for (int sb = wave; sb < NB; sb += WV) {
+    uint32_t wr[2][5];
+    side_words<KQ>(swa, c, wr[0]);
+    side_words<KQ>(swb, c, wr[1]);
+    const int nsb = sb + WV;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {  // the super-block's 8 chunks
-      if (j < 5 || nsb < NB) {
-        const int kn = j < 5 ? sb * 8 + j + 3 : nsb * 8 + j - 5;
-        load_q(kn, qa[(j + 3) & 3], qb[(j + 3) & 3]);
-        load_x(kn, xr[(j + 3) & 3]);
+      if (j < 9 - RD || nsb < NB) {
+        const int kn = j < 9 - RD ? sb * 8 + j + RD - 1 : nsb * 8 + j - (9 - RD);
+        load_q(kn, qa[(j + RD - 1) % RD], qb[(j + RD - 1) % RD]);
+        load_x(kn, xr[(j + RD - 1) % RD]);
+      }
+      if (j == 5 && nsb < NB) {  // the next super-block's records (from the start they would cost 10 registers more)
+        side_fetch<KQ>(rs, vs, nsb * (64 * SB), swa);
+        side_fetch<KQ>(rs, vs + 32 * SB, nsb * (64 * SB), swb);
       }
       __builtin_amdgcn_sched_barrier(0);  // keep the loads issued here, ahead of this chunk's products
-      const u32x4 ca = qa[j & 3], cb = qb[j & 3];
-      const u32x4* xc = xr[j & 3];
-      f16x16 dA = {}, dB = {};
+      const u32x4 ca = qa[j % RD], cb = qb[j % RD];
+      const u32x4* xc = xr[j % RD];
+      f16x16 d[2][TT] = {};
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
-        if (Q6 && st == 1) {
-          dA = f16x16{};
-          dB = f16x16{};
-        }
         const uint2 a0 = grid16(ca[2 * st]), a1 = grid16(ca[2 * st + 1]);
         const uint2 b0 = grid16(cb[2 * st]), b1 = grid16(cb[2 * st + 1]);
-        const h8v wva = __builtin_bit_cast(h8v, make_uint4(a0.x, a0.y, a1.x, a1.y));
-        const h8v wvb = __builtin_bit_cast(h8v, make_uint4(b0.x, b0.y, b1.x, b1.y));
-        const h8v xh = __builtin_bit_cast(h8v, xc[st]), xl = __builtin_bit_cast(h8v, xc[2 + st]);
-        dA = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, wva, dA, 0, 0, 0);
-        dB = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh, wvb, dB, 0, 0, 0);
-        dA = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, wva, dA, 0, 0, 0);
-        dB = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl, wvb, dB, 0, 0, 0);
+        const h8v w[2] = {__builtin_bit_cast(h8v, make_uint4(a0.x, a0.y, a1.x, a1.y)),
+                          __builtin_bit_cast(h8v, make_uint4(b0.x, b0.y, b1.x, b1.y))};
+#pragma unroll
+        for (int b = 0; b < TT; ++b)
+#pragma unroll
+          for (int a = 0; a < 2; ++a) {
+            if (Q6 && st == 1) d[a][b] = f16x16{};
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+              d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, xc[4 * b + 2 * half + st]), w[a], d[a][b], 0, 0, 0);
+          }
         if (Q6 || st == 1) {  // the sub-block is in: fold it
           const int js = Q6 ? 2 * j + st : j;
-          const float sa = sub_scale(wa, js), sbb = sub_scale(wb, js);
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            totA[r] = fmaf(sa, dA[r], totA[r]);
-            totB[r] = fmaf(sbb, dB[r], totB[r]);
+          for (int a = 0; a < 2; ++a) {
+            const float sc = sub_scale(wr[a], js);
+#pragma unroll
+            for (int b = 0; b < TT; ++b) {
+#pragma unroll
+              for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(sc, d[a][b][r], tot[a][b][r]);
+              // keep the fold here: sunk below the chunk loop's branches it would hold every chunk's tiles live (spills)
+              asm volatile("" : "+v"(tot[a][b]));
+            }
           }
-          // keep the fold here: sunk below the chunk loop's branches it would hold every chunk's tiles live (spills)
-          asm volatile("" : "+v"(totA), "+v"(totB));
+          if (Q6 && TT > 1) __builtin_amdgcn_sched_barrier(0);  // (else the next step's operands spill)
         }
       }
     }
-  }
-  __shared__ float part[GEMM_WAVES][2][16][64];
+    if (WV < 8 && --left == 0 && nsb < NB) {
+      aside = true;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    part[wave][0][r][lane] = totA[r];
-    part[wave][1][r][lane] = totB[r];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < 2 * 16 * 64; e += 64 * GEMM_WAVES) {
-    const int half = e >> 10, r = (e >> 6) & 15, l = e & 63;
-    float acc = 0.f;
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int w = 0; w < GEMM_WAVES; ++w) acc += part[w][half][r][l];
-    const int t = tt * 32 + 8 * (r / 4) + 4 * (l >> 5) + (r % 4);
-    if (t < m) Y[(size_t)t * ldy + row0 + rp * 64 + 32 * half + (l & 31)] = acc;
+        for (int b = 0; b < TT; ++b) {
+#pragma unroll
+          for (int r = 0; r < 16; r += 4)
+            own[(a + 2 * b) * 256 + r * 16] = f4v{tot[a][b][r], tot[a][b][r + 1], tot[a][b][r + 2], tot[a][b][r + 3]};
+          tot[a][b] = f16x16{};
+        }
+    }
   }
+  if (aside) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < TT; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          const f4v v = own[(a + 2 * b) * 256 + r * 16];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) tot[a][b][r + k] += v[k];
+        }
+  }
+  store_tiles<TT, WV>(tot, part, wave, lane, row0 + rp * 64, tt, m, Y, ldy);
+}
+
+template <int KQ, int TT, int WV>
+static hipError_t gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int nrows, const uint16_t* x, const uint16_t* sx,
+                               int m, float* Y, int ldy, hipStream_t s) {
+  const dim3 grid(nrows / 64, (m + 32 * TT - 1) / (32 * TT)), block(64 * WV);
+  const size_t smem = (size_t)WV * 2 * TT * 16 * 64 * 4;
+  if constexpr (KQ == KQ_Q4_K || KQ == KQ_Q5_K) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_prefill<KQ, TT, WV>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_gemm_prefill<KQ, TT, WV>), grid, block, smem, s, M, CT, row0, x, sx, m, Y, ldy);
+  } else {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_prefill_sub<KQ, TT, WV>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_gemm_prefill_sub<KQ, TT, WV>), grid, block, smem, s, M, CT, row0, x, m, Y, ldy);
+  }
+  return hipGetLastError();
+}
+
+template <int KQ>
+static hipError_t gemm_prefill_any(const DevMat& M, const uint8_t* CT, int row0, int nrows, const uint16_t* x,
+                                   const uint16_t* sx, int m, float* Y, int ldy, hipStream_t s) {
+  // 64 x 64 tiles per wave where they make 192 blocks (3/4 of the CUs), else 64 x 32; the K split over 4 waves where the
+  // blocks are more than the CUs, else over 8: us per call (preparation included) with 64 x 64 by 4 waves / by 8 / 64 x 32
+  // by 4 / by 8: Q4_K 14336 x 4096, m = 64 (224 blocks of 64 x 64) 38.6 / 37.9 / 41.2 / 45.7, m = 128 53 / 56 / 61 / 70,
+  // m = 2048 528 / 581 / 651 / 728; 4096 x 4096, m = 128 (128) 27.5 / 26.4 / 22.0 / 23.1, m = 512 (512) 46 / 48 / 50 / 61;
+  // 1024 x 4096, m = 128 (32) 25.1 / 23.8 / 19.0 / 18.3; Q6_K 4096 x 14336, m = 512 (512) 170 / 171 / 190 / 200. (By the
+  // matrix's rows, not the chunk's.)
+  const long long rows64 = M.N / 64, b64 = rows64 * ((m + 63) / 64), b32 = rows64 * ((m + 31) / 32);
+  if (b64 > 256) return gemm_prefill<KQ, 2, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+  if (b64 >= 192) return gemm_prefill<KQ, 2, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+  if (b32 >= 256) return gemm_prefill<KQ, 1, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+  return gemm_prefill<KQ, 1, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
 }
 
 hipError_t launch_gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int nrows, const void* XT,
                                const void* SXT, int m, float* Y, int ldy, hipStream_t s) {
   if (nrows < 1 || m < 1 || nrows % 64 || M.K % 256) return hipErrorInvalidValue;
-  const dim3 grid(nrows / 64, (m + 31) / 32), block(64 * GEMM_WAVES);
   const uint16_t* x = static_cast<const uint16_t*>(XT);
   const uint16_t* sx = static_cast<const uint16_t*>(SXT);
   switch (M.kqt) {
-    case KQ_Q4_K: hipLaunchKernelGGL(k_gemm_prefill<KQ_Q4_K>, grid, block, 0, s, M, CT, row0, x, sx, m, Y, ldy); break;
-    case KQ_Q5_K: hipLaunchKernelGGL(k_gemm_prefill<KQ_Q5_K>, grid, block, 0, s, M, CT, row0, x, sx, m, Y, ldy); break;
-    case KQ_Q6_K: hipLaunchKernelGGL(k_gemm_prefill_sub<KQ_Q6_K>, grid, block, 0, s, M, CT, row0, x, m, Y, ldy); break;
-    case KQ_IQ4_XS: hipLaunchKernelGGL(k_gemm_prefill_sub<KQ_IQ4_XS>, grid, block, 0, s, M, CT, row0, x, m, Y, ldy); break;
+    case KQ_Q4_K: return gemm_prefill_any<KQ_Q4_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case KQ_Q5_K: return gemm_prefill_any<KQ_Q5_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case KQ_Q6_K: return gemm_prefill_any<KQ_Q6_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case KQ_IQ4_XS: return gemm_prefill_any<KQ_IQ4_XS>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 }  // namespace lw

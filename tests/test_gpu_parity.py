@@ -943,3 +943,26 @@ def test_gpu_model_shaped_bundle(gpu, tmp_path, orc):
                   first[0] + " within budget")
         with pytest.raises(RuntimeError, match="not resident"):
             rt.test_matmul(last[0], np.zeros((1, last[3]), np.float32))
+
+
+@pytest.mark.parametrize("kqt,K", [(1, 1024), (2, 768), (3, 768), (4, 1024)])
+def test_gpu_prefill_tile_shapes(gpu, tmp_path, orc, kqt, K):
+    """The prefill GEMM's block shapes at their edges: 64 x 64 tiles by 4 waves (from 192 blocks: 192 x 64 rows and one
+    token tile pair, ragged token counts, three pairs), 64 x 32 tiles by 4 waves (from 256 blocks) and by 8 below, with
+    fewer super-blocks than waves. The tolerance is the fp32 sums' (2-norm), far below a wrong tile or scale."""
+    import torch
+    from lazyweights_amd import Runtime, bundle
+    mats = [("p%d" % N, kqt, N, K, {1: 2.3, 2: 3.4, 3: 4.3, 4: 2.6}[kqt], 700 + N) for N in (64, 4096, 12288)]
+    bundle.write_synthetic_bundle(str(tmp_path), mats, threads=16)
+    with Runtime(tmp_path) as rt:
+        for name, _, N, _, H, seed in mats:
+            w = orc.dequant(kqt, *bundle.synth_matrix(kqt, N, K, H, seed, threads=16))
+            for m in {64: (9, 33, 130), 4096: (97, 128, 129), 12288: (9, 64, 65, 131)}[N]:
+                x = torch.randn(m, K, generator=torch.Generator().manual_seed(m))
+                y = torch.full((m, N), float("nan"), device="cuda")
+                rt.matmul_dev(name, x.cuda(), y, x_f16=False)
+                torch.cuda.synchronize()
+                y64 = x.double().numpy() @ w.astype(np.float64).T
+                e = np.linalg.norm(y.double().cpu().numpy() - y64) / np.linalg.norm(y64)
+                say("prefill tiles", name, kqt, "m", m, "err %.2g" % e)
+                assert e < 1e-6
