@@ -72,7 +72,7 @@ struct WideUnit {
   static constexpr int NST = RUN / 8;    // products per run
   static constexpr int PPS = 16 / NST;   // pairs of symbols per product
   static constexpr int XD = 2;           // products (of both passes) whose activations are in flight
-  static constexpr int NA = 2 * NSB;     // accumulators: a super-block of a row each (index 2 sb + i)
+  static constexpr int NA = 2 * NSB;     // side records: a super-block of a row each (index 2 sb + i)
   // chain starts; side records as loaded (Q6_K: d and the scales of the run's sub-blocks of both passes)
   uint32_t start[4], raw[NA][5];
   u32x4 x[XD][2], sx[NSB];
@@ -162,9 +162,21 @@ struct WideUnit {
     }
     const uint32_t rlb =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint32_t*)(buf + (lane & 15));
-    f4v acc[NA];
+    // sums of a chain (Q5_K, for the registers: of a row's two), folded into tot every 16 symbols of the 8-bit formats (one
+    // run of additions over 256 weights was 1.3 .. 1.6 times as far from 64 bits)
+    constexpr int NACC = KQ == KQ_Q5_K ? 2 : 4;
+    f4v acc[NACC];
 #pragma unroll
-    for (int a = 0; a < NA; ++a) acc[a] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NACC; ++c) acc[c] = f4v{0.f, 0.f, 0.f, 0.f};
+    auto fold = [&]() {
+#pragma unroll
+      for (int c = 0; c < NACC; ++c) {
+        const float d = h2f(d2[NSB == 2 ? c >> 1 : 0] >> (16 * (c & 1))) * WSCALE;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tot[c & 1][r] = fmaf(d, acc[c][r], tot[c & 1][r]);
+        acc[c] = f4v{0.f, 0.f, 0.f, 0.f};
+      }
+    };
     // P form: bit position in the buffer - GUARD_BITS + 64; slot = P >> 5 is the window row after the two in A and B
     uint32_t P[4], slot[4], A[4], B[4], C[4];
 #pragma unroll
@@ -237,7 +249,7 @@ struct WideUnit {
           };
           const uint32_t v0 = scaled(w4[c][0]), v1 = scaled(w4[c][1]);
           const u32x4 xp = x[st % XD][c >> 1];
-          f4v& a = acc[NSB == 2 ? c : c & 1];
+          f4v& a = acc[c % NACC];
           a = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4v, make_uint2(xp[2 * h], xp[2 * h + 1])),
                                                     __builtin_bit_cast(h4v, make_uint2(v0, v1)), a, 0, 0, 0);
         };
@@ -248,14 +260,10 @@ struct WideUnit {
           for (int c = 0; c < 4; ++c) product(c, s0[c], n0[c]);
         }
         if constexpr (q % PPS == PPS - 1 && st + XD < NST) load_x(st + XD);
+        if constexpr (SYMB == 8 && q != 15 && q % (KQ == KQ_Q5_K ? 4 : 8) == (KQ == KQ_Q5_K ? 3 : 7)) fold();
       }
     });
-#pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      const float d = h2f(d2[a / 2] >> (16 * (a & 1))) * WSCALE;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(d, acc[a][r], tot[a & 1][r]);
-    }
+    fold();
   }
 };
 
