@@ -75,9 +75,20 @@ __global__ void __launch_bounds__(256) k_prefill_prep(DevMat M, uint8_t* __restr
   const int t = tr0 * KT + (int)blockIdx.x - px.blocks;
   const int tc = t % KT, tr = t / KT;
   const int R = min((int)M.rows[t] + 2, stage_rows);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l = lane & 31, f = lane >> 5;
+  // the tile's rows, 8 per direct-to-LDS load, the waves in turn, and the table: every load in flight at once (through
+  // registers in a loop each turn waited for its own: 4096 x 4096 with m = 128 9.8 us, so 8.1; 14336 x 4096 18.7 and 15.5)
+  const uint4* src = reinterpret_cast<const uint4*>(M.words + M.tbase[t]) + lane;
+  for (int i = wave; 8 * i < R; i += 4)
+    if (lane < 8 * (R - 8 * i))
+      __builtin_amdgcn_global_load_lds(src + 64 * i, (__attribute__((address_space(3))) void*)(tw + 256 * i), 16, 0, 0);
   if (SYMB == 4) {  // entries len | grid byte of the pair's first code << 16 | second << 24 (decode_table4)
-    for (int i = threadIdx.x; i < LUTN / 4; i += 256)
-      reinterpret_cast<uint4*>(lut4)[i] = reinterpret_cast<const uint4*>(M.lut4)[i];
+    const uint4* ta = reinterpret_cast<const uint4*>(M.lut4) + lane;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds(ta + 64 * (wave + 4 * i),
+                                       (__attribute__((address_space(3))) void*)(lut4 + 256 * (wave + 4 * i)), 16, 0, 0);
   } else {  // sym | len << 8 -> len | sym << 16, 8 entries a thread
     static_assert(LUTN == 8 * 256, "8 entries per thread");
     const uint4 v = reinterpret_cast<const uint4*>(M.lut)[threadIdx.x];
@@ -86,11 +97,6 @@ __global__ void __launch_bounds__(256) k_prefill_prep(DevMat M, uint8_t* __restr
     o[0] = make_uint4(entry(v.x), entry(v.x >> 16), entry(v.y), entry(v.y >> 16));
     o[1] = make_uint4(entry(v.z), entry(v.z >> 16), entry(v.w), entry(v.w >> 16));
   }
-  const uint4* src = reinterpret_cast<const uint4*>(M.words + M.tbase[t]);
-  for (int i = threadIdx.x; i < 8 * R; i += 256) reinterpret_cast<uint4*>(tw)[i] = src[i];
-  __syncthreads();
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, l = lane & 31, f = lane >> 5;
   const int k = 4 * f + wave;  // segment of bit-lane l: row f * 32 + l, symbols 64 wave .. 64 wave + 63
   const uint32_t tsel = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint32_t*)lut4;
   uint32_t tmask = 0x1FFCu;
@@ -98,8 +104,11 @@ __global__ void __launch_bounds__(256) k_prefill_prep(DevMat M, uint8_t* __restr
   const uint32_t rlb = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)(tw + l);
   uint32_t P[2], slot[2], A[2], B[2], C[2];
 #pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
+  for (int ch = 0; ch < 2; ++ch)
     P[ch] = (uint32_t)M.split[((size_t)t * SPLITS + 2 * k + ch) * 32 + (uint32_t)l] - GUARD_BITS + 64u;
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int ch = 0; ch < 2; ++ch) {
     slot[ch] = __builtin_amdgcn_ubfe(P[ch], 5, 8);
     A[ch] = *(LdsU32*)(rlb + ((slot[ch] - 2u) << 7));
     B[ch] = *(LdsU32*)(rlb + ((slot[ch] - 1u) << 7));
