@@ -18,13 +18,13 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <fstream>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <sstream>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -144,6 +144,7 @@ struct Model {
   size_t dec_cap = 0;
   uint8_t* pin = nullptr;
   hipEvent_t pin_ev[kPieces] = {};
+  std::mutex dec_mu;  // held by the call that uses them
   int verbose = 0;
   Tensor* find(const char* name) {
     if (!name) return nullptr;
@@ -1522,10 +1523,11 @@ uint8_t* scratch_on_device() {
 constexpr int kCopyThreads = 4;
 int copy_out(Model& M, uint8_t* out, const uint8_t* src, size_t n) {
   if (!M.pin && hipHostMalloc(reinterpret_cast<void**>(&M.pin), kPieces * kPieceBytes) != hipSuccess) {
-    M.pin = nullptr;
+    M.pin = nullptr;  // no pinned memory to be had: the plain copy
     (void)hipGetLastError();
-    g_err = "pinned host allocation failed";
-    return -1;
+    HIPCHECK(hipStreamSynchronize(M.stream));
+    HIPCHECK(hipMemcpy(out, src, n, hipMemcpyDeviceToHost));
+    return 0;
   }
   for (hipEvent_t& e : M.pin_ev)
     if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -1569,7 +1571,7 @@ int copy_out(Model& M, uint8_t* out, const uint8_t* src, size_t n) {
   if (pieces > 1) {
     try {
       for (int i = 0; i < std::min(kCopyThreads, pieces); ++i) threads.emplace_back(worker);
-    } catch (const std::system_error&) {  // fewer threads, or none: this one takes what is left below
+    } catch (const std::exception&) {  // fewer threads, or none: this one takes what is left below
     }
   }
   for (; q < pieces && error.load() == hipSuccess; ++q) {  // a slot is free once its last piece is copied out
@@ -1787,13 +1789,19 @@ int rt_test_decode(void* h, const char* name, uint8_t* out) {
     g_err = t->name + ": not resident";
     return -1;
   }
-  const int rows = (int)std::max<size_t>(1, kDecodeDevBytes / ((size_t)lw::TN * t->K));  // tile rows at a time
-  for (int tr0 = 0; tr0 < t->dm.NT; tr0 += rows) {
-    const int tr1 = std::min(t->dm.NT, tr0 + rows);
-    const size_t bytes = (size_t)(tr1 - tr0) * lw::TN * t->K;
-    if (grow(M->dec, M->dec_cap, bytes)) return -1;
-    HIPCHECK(lw::launch_decode(t->dm, M->dec, tr0, tr1, M->stream));
-    if (copy_out(*M, out + (size_t)tr0 * lw::TN * t->K, M->dec, bytes)) return -1;
+  try {  // (the piece table and the threads' handles are allocated)
+    std::lock_guard<std::mutex> lk(M->dec_mu);
+    const int rows = (int)std::max<size_t>(1, kDecodeDevBytes / ((size_t)lw::TN * t->K));  // tile rows at a time
+    for (int tr0 = 0; tr0 < t->dm.NT; tr0 += rows) {
+      const int tr1 = std::min(t->dm.NT, tr0 + rows);
+      const size_t bytes = (size_t)(tr1 - tr0) * lw::TN * t->K;
+      if (grow(M->dec, M->dec_cap, bytes)) return -1;
+      HIPCHECK(lw::launch_decode(t->dm, M->dec, tr0, tr1, M->stream));
+      if (copy_out(*M, out + (size_t)tr0 * lw::TN * t->K, M->dec, bytes)) return -1;
+    }
+  } catch (const std::exception& e) {
+    g_err = std::string("rt_test_decode: ") + e.what();
+    return -1;
   }
   return 0;
 }

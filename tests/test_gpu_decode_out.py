@@ -20,3 +20,17 @@ def test_codes_reach_the_host(gpu, lib, tmp_path, kqt, N, K):
         for _ in range(2):
             assert lib.rt_test_decode(rt.h, b"a", out.ctypes.data) == 0
         assert np.array_equal(out[:N], a) and (out[N] == 0xAA).all()
+
+
+def test_two_threads_on_one_handle(gpu, lib, tmp_path):
+    """Calls that overlap on one handle take its kept buffers in turn."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from lazyweights_amd import Runtime, bundle
+    mats = [("a", 1, 1024, 4096, 2.3, 51), ("b", 3, 2112, 1024, 4.3, 52)]
+    bundle.write_synthetic_bundle(str(tmp_path), mats, threads=16)
+    want = {m[0]: bundle.synth_matrix(*m[1:], threads=16)[0] for m in mats}
+    with Runtime(tmp_path) as rt, ThreadPoolExecutor(2) as pool:
+        got = list(pool.map(lambda n: (n, rt.test_decode(n)), ["a", "b"] * 4))
+        for name, codes in got:
+            assert np.array_equal(codes, want[name])
