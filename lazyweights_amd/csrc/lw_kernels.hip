@@ -3741,7 +3741,7 @@ __global__ void __launch_bounds__(256) k_unpack(DevMat M, uint8_t* __restrict__ 
   const int tc = (int)(tt % M.KT), trr = (int)(tt / M.KT);
   const uint4 c = reinterpret_cast<const uint4*>(M.words)[((size_t)(tr0 + trr) * M.KT + tc) * 1024 + (size_t)(g * 64 + L)];
   const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-  if (TILED) {  // the prefill GEMM's layout (launch_decode_tiled): 16 codes (IQ4_XS: grid bytes) per 16-byte piece
+  if (TILED) {  // the prefill GEMM's layout (launch_prefill_prep): 16 codes (IQ4_XS: grid bytes) per 16-byte piece
     const int row = trr * TN + L, KC = M.K / 32;
     uint8_t* o = out + ((size_t)(row >> 5) * KC * 64 + (row & 31)) * 16;
     if (SYMB == 4) {  // 32 codes = one chunk: symbols 0..7 -> piece h = 0, 8..15 -> h = 1

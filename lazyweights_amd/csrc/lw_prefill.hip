@@ -54,7 +54,7 @@ __device__ __forceinline__ void prefill_x_block(const PrefillX& px, int block) {
 }
 
 
-// Codes in the prefill GEMM's tiled layout (launch_decode_tiled): one block of 4 waves per tile as k_decode_split,
+// Codes in the prefill GEMM's tiled layout (launch_prefill_prep): one block of 4 waves per tile as k_decode_split,
 // but each lane runs the two 32-symbol chains of its 64-symbol segment (split starts 2k and 2k + 1) interleaved, and
 // stores its codes straight from registers: 16 codes make one lane's piece of the tiled layout, and the 32 lanes of a
 // row half write 32 consecutive pieces (512 B) per store. No code rows in LDS: the block holds the table and the tile.
@@ -205,7 +205,7 @@ hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, 
 // the scaling of codes per product). 64 x 64 tiles take all 256 registers of 2 waves per SIMD (128 in accumulators): the
 // operand rings are 2 chunks deep instead of 4, side records and x sums are read through buffers (no per-lane addresses)
 // half a super-block ahead, and a tile's registers take its mins product once it is folded. Q4_K 14336 x 4096, m = 2048:
-// 728 -> 516 us with the preparation, 496 useful TFLOP/s in the GEMM = 992 of products, where a library fp16 GEMM of
+// 728 -> 516 us with the preparation (526 with the totals put aside, below), 496 useful TFLOP/s in the GEMM = 992 of products, where a library fp16 GEMM of
 // 8192 x 8192 x 8192 reaches 1176 on this card.
 // codes q0..q3 (bytes of qw) -> sc q / 16 as 4 fp16 in two words (nsc = -64 sc)
 __device__ __forceinline__ uint2 scaled_codes16(uint32_t qw, h2v sc, h2v nsc) {
@@ -323,6 +323,34 @@ __device__ __forceinline__ void store_tiles(const f16x16 (&tot)[2][TT], float* p
   }
 }
 
+// A wave's totals to its part of the LDS (own: [tile][r / 4][lane]) and zero again, and added back.
+template <int TT>
+__device__ __forceinline__ void put_aside(f16x16 (&tot)[2][TT], f4v* own) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b) {
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        own[(a + 2 * b) * 256 + r * 16] = f4v{tot[a][b][r], tot[a][b][r + 1], tot[a][b][r + 2], tot[a][b][r + 3]};
+      tot[a][b] = f16x16{};
+    }
+}
+
+template <int TT>
+__device__ __forceinline__ void take_back(f16x16 (&tot)[2][TT], const f4v* own) {
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4) {
+        const f4v v = own[(a + 2 * b) * 256 + r * 16];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) tot[a][b][r + k] += v[k];
+      }
+}
+
 template <int KQ, int TT, int WV>
 __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, const uint8_t* __restrict__ CT, int row0,
                                                                      const uint16_t* __restrict__ XT,
@@ -362,6 +390,12 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
         x[4 * b + i] = __builtin_amdgcn_raw_buffer_load_b128(rx, vo + i * 1024, (b * KC + kc) * 4096, 0);
   };
   f16x16 tot[2][TT] = {};
+  extern __shared__ float part[];
+  // with 4 waves sharing K the totals are put aside half way, as in k_gemm_prefill_sub: 14336 x 4096, m = 2048 1.8e-7
+  // from 64 bits without, 1.7e-7 with 8 waves and with this, which takes 512 -> 526 us (6 registers spill around it)
+  int left = WV < 8 ? ((NB - wave + WV - 1) / WV + 1) / 2 : 0;
+  bool aside = false;
+  f4v* const own = reinterpret_cast<f4v*>(part) + wave * 2 * TT * 256 + lane;
   uint32_t swa[5] = {}, swb[5] = {};
   u32x4 qa[RD] = {}, qb[RD] = {}, xr[RD][4 * TT] = {};
   if (wave < NB) {
@@ -438,8 +472,12 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
         for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(-dmin, d[a][b][r], tot[a][b][r]);
       }
     }
+    if (WV < 8 && --left == 0 && nsb < NB) {
+      aside = true;
+      put_aside<TT>(tot, own);
+    }
   }
-  extern __shared__ float part[];
+  if (aside) take_back<TT>(tot, own);
   store_tiles<TT, WV>(tot, part, wave, lane, row0 + rp * 64, tt, m, Y, ldy);
 }
 
@@ -594,29 +632,10 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill_sub(DevMat
     }
     if (WV < 8 && --left == 0 && nsb < NB) {
       aside = true;
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < TT; ++b) {
-#pragma unroll
-          for (int r = 0; r < 16; r += 4)
-            own[(a + 2 * b) * 256 + r * 16] = f4v{tot[a][b][r], tot[a][b][r + 1], tot[a][b][r + 2], tot[a][b][r + 3]};
-          tot[a][b] = f16x16{};
-        }
+      put_aside<TT>(tot, own);
     }
   }
-  if (aside) {
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < TT; ++b)
-#pragma unroll
-        for (int r = 0; r < 16; r += 4) {
-          const f4v v = own[(a + 2 * b) * 256 + r * 16];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) tot[a][b][r + k] += v[k];
-        }
-  }
+  if (aside) take_back<TT>(tot, own);
   store_tiles<TT, WV>(tot, part, wave, lane, row0 + rp * 64, tt, m, Y, ldy);
 }
 
