@@ -205,8 +205,8 @@ hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, 
 // the scaling of codes per product). 64 x 64 tiles take all 256 registers of 2 waves per SIMD (128 in accumulators): the
 // operand rings are 2 chunks deep instead of 4, side records and x sums are read through buffers (no per-lane addresses)
 // half a super-block ahead, and a tile's registers take its mins product once it is folded. Q4_K 14336 x 4096, m = 2048:
-// 728 -> 516 us with the preparation (526 with the totals put aside, below), 496 useful TFLOP/s in the GEMM = 992 of products, where a library fp16 GEMM of
-// 8192 x 8192 x 8192 reaches 1176 on this card.
+// 728 -> 516 us with the preparation (526 with the totals put aside, below), 496 useful TFLOP/s in the GEMM = 992 of
+// products, where a library fp16 GEMM of 8192 x 8192 x 8192 reaches 1176 on this card.
 // codes q0..q3 (bytes of qw) -> sc q / 16 as 4 fp16 in two words (nsc = -64 sc)
 __device__ __forceinline__ uint2 scaled_codes16(uint32_t qw, h2v sc, h2v nsc) {
   const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x54545454u, qw, 0x04010400u));
