@@ -377,7 +377,10 @@ k_fused_wide(WidePlan plan, int buf_rows) {
       __hip_atomic_store(e->P + ((size_t)part * mo + tok) * N + o, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (np == 1) return;
-  // the block that counts the row's last part sums the parts in order
+  // the block that counts the row's last part sums the parts in order; it counts its own once every wave's partials are
+  // stored (a workgroup barrier alone does not wait for global stores)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
   if (threadIdx.x == 0) {
     const uint32_t old = __hip_atomic_fetch_add(e->cnt + hr0, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (old == (uint32_t)(np - 1)) {

@@ -1,7 +1,15 @@
 """The build's DPP wait-state check (lazyweights_amd/build.py dpp_violations) on hand-written disassembly: the
 hazards it must refuse and the forms it must accept (the check guards the inline-assembly DPP products, which the
-compiler's hazard recognizer does not see)."""
-from lazyweights_amd.build import dpp_violations
+compiler's hazard recognizer does not see); and properties of the built kernels that no run shows reliably."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from lazyweights_amd import _lib
+from lazyweights_amd.build import ARCH, OBJDUMP, dpp_violations
 
 HEAD = "0000000000001000 <k>:\n"
 
@@ -64,3 +72,36 @@ def test_mfma_write_of_the_dpp_source_needs_the_matrix_core_wait():
     assert dpp_violations(body(*pad, mfma, "s_nop 7", "s_nop 7", DPP))  # 16
     assert not dpp_violations(body(*pad, mfma, "s_nop 7", "s_nop 7", "s_nop 2", DPP))  # 19
     assert not dpp_violations(body(*pad, "v_mfma_f32_4x4x4_16b_f16 v[8:11], v[0:1], v[2:3], v[8:11]", DPP))
+
+
+@pytest.fixture(scope="module")
+def kernels(lib, tmp_path_factory):
+    """The built library's gfx950 code objects: a function (symbol pattern) -> {mangled name: (object path)}."""
+    d = tmp_path_factory.mktemp("objs")
+    shutil.copy(_lib.LIB_PATH, d / "l.so")
+    subprocess.run([OBJDUMP, "--offloading", "l.so"], cwd=d, check=True, stdout=subprocess.DEVNULL)
+    objs = {str(d / f): subprocess.run([OBJDUMP, "-t", f], cwd=d, check=True, text=True, stdout=subprocess.PIPE).stdout
+            for f in os.listdir(d) if ARCH in f}
+
+    def find(pattern):
+        return {m.group(1): obj for obj, table in objs.items()
+                for m in re.finditer(r"F \.text\s+\S+(?: \.\w+)? (\S*%s\S*)$" % pattern, table, re.M)}
+    return find
+
+
+def test_wide_kernel_counts_a_row_after_every_waves_stores(kernels):
+    """A block of k_fused_wide counts its part of a row only after all its waves' partials are stored: between the last
+    store and the counter's increment every wave waits for its stores and meets the others at a barrier."""
+    found = kernels("k_fused_wide")
+    assert found
+    for name, obj in found.items():
+        text = subprocess.run([OBJDUMP, "-d", "--mcpu=" + ARCH, "--disassemble-symbols=" + name, obj], check=True, text=True,
+                              stdout=subprocess.PIPE).stdout
+        ops = [m.group(1) for m in re.finditer(r"^\t((?:global_store|global_atomic_add|s_barrier|s_waitcnt)\S*.*?)\s*//", text,
+                                               re.M)]
+        adds = [i for i, op in enumerate(ops) if op.startswith("global_atomic_add")]
+        assert len(adds) == 1, name
+        before = ops[:adds[0]]
+        after_store = before[max(i for i, op in enumerate(before) if op.startswith("global_store")) + 1:]
+        wait = next((i for i, op in enumerate(after_store) if "vmcnt(0)" in op), None)
+        assert wait is not None and "s_barrier" in after_store[wait:], name
