@@ -21,6 +21,7 @@ typedef int v4i32 __attribute__((ext_vector_type(4)));
 typedef float f16x16 __attribute__((ext_vector_type(16)));
 
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef __bf16 b8v __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float h2f(uint32_t bits16) {

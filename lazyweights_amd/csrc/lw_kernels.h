@@ -180,7 +180,7 @@ struct WidePlan {
 constexpr int WIDE_MAX_WAVES = 16;
 size_t wide_x_bytes(int mt, int K);  // bytes of one reordered vector
 // activations for it in one launch: job i reorders X[i] (fp16 [mt][K], any alignment; per = 2: fp32 [mt / 2][K], split
-// into hi + lo) into XT[i] (mt K fp16, 16-byte aligned)
+// into hi + lo) into XT[i] (wide_x_bytes(mt, K[i]) bytes, 16-byte aligned: mt K fp16, then the sub-blocks' sums)
 struct WideXJobs {
   const void* X[MAX_GROUP];
   void* XT[MAX_GROUP];

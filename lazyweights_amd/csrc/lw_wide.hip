@@ -25,7 +25,9 @@
 //   and s0 f(q) are exact and both products go to one accumulator; IQ4_XS's kv / 16 = fp16(64 + b / 16) - 72 of the grid
 //   byte b = kv + 128, one fma per product.
 // d is applied in fp32 when the super-block is complete. Mins (Q4_K / Q5_K): one product per row group and super-block of
-// the mins with the sub-blocks' x sums (fp16 hi and lo halves, formed by launch_wide_x).
+// the mins with the sub-blocks' fp32 x sums, formed by launch_wide_x and held as three bf16 parts that add up to all 24
+// bits (as fp16 hi and lo a sum past 65504, 32 activations of 2047, would be infinite): parts in lane groups 0, 1 and 2 of
+// v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16.
 // Distance from 64 bits 1.3e-7 (2-norm), against 3e-6 of the ring kernel's fp16 dot products and 2e-7 .. 8e-7 of
 // k_fused_tiles_mma.
 //
@@ -107,15 +109,15 @@ struct WideUnit {
     for (int c = 0; c < 4; ++c)
       start[c] = M.hsplit[(((size_t)t * 2 + (uint32_t)f) * 64 + 32 * (c >> 1) + 16 * (c & 1)) * 4 + (uint32_t)(4 * j + g)];
     const int xbytes = 2 * mt * K;
-    xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(e->X), (short)0, xbytes + xbytes / 16, kBufferRsrcWord3);
+    xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(e->X), (short)0, xbytes + xbytes / 32 * 3, kBufferRsrcWord3);
     xv = j < mt ? (uint32_t)(16 * (g * mt + j)) : 0x7FFFFFF0u;
     x0 = tc * 2 * NST * 64 * mt;
     xs = 64 * mt;
-    // lanes g = 0 the hi, g = 1 the lo halves of a super-block's 8 x sums
+    // lanes g < 3 part g of a super-block's 8 x sums
     if constexpr (MINS) {
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
-        sx[sb] = __builtin_amdgcn_raw_buffer_load_b128(xr, g < 2 ? xv : 0x7FFFFFF0u, xbytes + (NSB * tc + sb) * 32 * mt, 0);
+        sx[sb] = __builtin_amdgcn_raw_buffer_load_b128(xr, g < 3 ? xv : 0x7FFFFFF0u, xbytes + (NSB * tc + sb) * 48 * mt, 0);
     }
 #pragma unroll
     for (int st = 0; st < XD; ++st) load_x(st);
@@ -151,11 +153,14 @@ struct WideUnit {
         }
         float mf[8];
         side_mins(w, mf);
-        const h8v m = {(_Float16)mf[0], (_Float16)mf[1], (_Float16)mf[2], (_Float16)mf[3],
-                       (_Float16)mf[4], (_Float16)mf[5], (_Float16)mf[6], (_Float16)mf[7]};
+        u32x4 m;  // as bf16, the upper halves
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          m[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, mf[2 * k + 1]), __builtin_bit_cast(uint32_t, mf[2 * k]),
+                                       0x07060302u);
         const float off = -h2f(w[0] >> 16);
-        const f4v ma = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, sx[a >> 1]), m,
-                                                              f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        const f4v ma = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, sx[a >> 1]), __builtin_bit_cast(b8v, m),
+                                                               f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(off, ma[r], tot[a & 1][r]);
       }
@@ -417,17 +422,20 @@ __global__ void __launch_bounds__(256) k_wide_x(WideXJobs q) {
   const int run8 = q.symbits[jb] == 4 ? 8 : 4;          // products per run
   const int st = c % run8, g = c / run8 % 4, piece = c / (4 * run8) * run8 + st;
   uint4* out = static_cast<uint4*>(q.XT[jb]) + (size_t)piece * 4 * mt + g * mt;
-  // the sum of the thread's 8, then of the sub-block's 32 (4 threads): its place in the super-block's 8 hi halves of
-  // each token, then 8 lo halves, after the pieces
+  // the sum of the thread's 8, then of the sub-block's 32 (4 threads), as three bf16 parts, each what is left cut to 8
+  // bits: its place in the super-block's 8 first parts of each token, then 8 second and 8 third ones, after the pieces
   uint16_t* sxo = reinterpret_cast<uint16_t*>(static_cast<uint4*>(q.XT[jb]) + (size_t)n8 * mt) +
-                  (size_t)(c / 32) * 16 * mt + (c >> 2 & 7);
+                  (size_t)(c / 32) * 24 * mt + (c >> 2 & 7);
   auto put_sum = [&](float a, int tk) {
     a += __shfl_xor(a, 1);
     a += __shfl_xor(a, 2);
     if (c & 3) return;
-    const _Float16 h = (_Float16)a;
-    sxo[8 * tk] = __builtin_bit_cast(uint16_t, h);
-    sxo[8 * (mt + tk)] = (uint16_t)f2h(a - (float)h);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint32_t u = __builtin_bit_cast(uint32_t, a) & 0xFFFF0000u;
+      sxo[8 * (k * mt + tk)] = (uint16_t)(u >> 16);
+      a -= __builtin_bit_cast(float, u);
+    }
   };
   auto sum8 = [&](const uint32_t* v) {
     float a = 0.f;
@@ -463,7 +471,7 @@ __global__ void __launch_bounds__(256) k_wide_x(WideXJobs q) {
   }
 }
 
-size_t wide_x_bytes(int mt, int K) { return (size_t)mt * K * 2 + (size_t)mt * K / 8; }
+size_t wide_x_bytes(int mt, int K) { return (size_t)mt * K * 2 + (size_t)mt * (K / 256) * 48; }
 
 hipError_t launch_wide_x(WideXJobs q, hipStream_t s) {
   if (q.n < 1 || q.n > MAX_GROUP || q.mt < 1 || q.mt > WIDE_TOKENS || (q.per != 1 && q.per != 2) || q.mt % q.per)

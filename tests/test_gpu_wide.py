@@ -112,3 +112,31 @@ def test_token_order_nan_and_scratch_limit(gpu, lib, orc, tmp_path):
         assert torch.equal(y, ref)
     finally:
         rt.close()
+
+
+@pytest.mark.parametrize("kqt", (1, 2))
+def test_sub_block_sums_past_fp16(gpu, lib, orc, tmp_path, kqt):
+    """The mins take the sums of 32 activations in the range and with the bits of fp32: sub-blocks of 3000 (a sum of 96000,
+    past fp16's largest number), two activations of 40000, and 32 of the largest fp16 number, beside ordinary ones. Measured
+    against sum |w x|, the size of the terms: fp32 sums of 16, so a few 2^-24."""
+    import torch
+    rt, w = open_mats(tmp_path, [("a", kqt, 192, 4608, H[kqt], 31)])
+    try:
+        d = orc.dequant(kqt, *w["a"])
+        for m, f16 in ((5, True), (9, True), (16, True), (1, False), (8, False)):
+            x = torch.randn(m, 4608, generator=torch.Generator().manual_seed(m))
+            x[0, 96:128] = 3000
+            x[m // 2, [512, 540]] = 40000
+            x[m - 1, 4576:] = -65504
+            x = (x.half() if f16 else x).cuda()
+            y = torch.full((m, 192), float("nan"), device="cuda")
+            assert lib.lw_matmul_dev(rt.h, b"a", x.data_ptr(), int(f16), m, y.data_ptr(), 192, None) == 0
+            torch.cuda.synchronize()
+            y = y.double().cpu().numpy()
+            x64 = x.float().cpu().double().numpy()
+            ref, size = orc.gemv_f64(d, x64), orc.gemv_f64(np.abs(d), np.abs(x64))
+            e = np.linalg.norm(y - ref, axis=1) / np.linalg.norm(size, axis=1)
+            print("sums", kqt, m, f16, "err %.2g" % e.max(), flush=True)
+            assert e.max() < TOL, (m, f16)
+    finally:
+        rt.close()
