@@ -6,8 +6,9 @@ namespace lw {
 // x of the prefill GEMM: fp32 X [m][K] -> XT (fp16 hi = fp16(x), lo = fp16(x - hi)) and SXT (per sub-block of 32
 // weights s = ((a0 + a1) + (a2 + a3)), a_q the in-order fp32 sum of its q-th 8 values, as fp16 hi / lo), tokens
 // padded with zeros to a multiple of 64. Thread = (chunk, q, token c of the tile): the 32 threads of one q write one
-// lane-linear 512-byte run of a piece; the chunk's four a_q meet in LDS.
-__device__ __forceinline__ void prefill_x_block(const PrefillX& px, int block) {
+// lane-linear 512-byte run of a piece; the chunk's four a_q meet in LDS (part: PREFILL_X_LDS floats).
+constexpr int PREFILL_X_LDS = 2 * 4 * 32;
+__device__ __forceinline__ void prefill_x_block(const PrefillX& px, int block, float* part) {
   const float* __restrict__ const X = px.X;
   uint16_t* __restrict__ const XT = px.XT;
   uint16_t* __restrict__ const SXT = px.SXT;
@@ -40,19 +41,17 @@ __device__ __forceinline__ void prefill_x_block(const PrefillX& px, int block) {
   o[0] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
   o[2 * 64] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
   if (!SXT) return;  // formats without mins
-  __shared__ float part[2][4][32];                       // the block's two chunks
-  const int cb = (threadIdx.x >> 7) & 1;
-  part[cb][q][c] = sum;
+  float* const p = part + ((threadIdx.x >> 7) & 1) * 128 + c;  // of the block's two chunks
+  p[32 * q] = sum;
   __syncthreads();
   if (q == 0) {
-    const float s = (part[cb][0][c] + part[cb][1][c]) + (part[cb][2][c] + part[cb][3][c]);
+    const float s = (p[0] + p[32]) + (p[64] + p[96]);
     const _Float16 hi = (_Float16)s;
     uint16_t* sx = SXT + ((((size_t)tt * NB + (kc >> 3)) * 2) * 32 + c) * 8 + (kc & 7);
     sx[0] = __builtin_bit_cast(uint16_t, hi);
     sx[32 * 8] = __builtin_bit_cast(uint16_t, (_Float16)(s - (float)hi));
   }
 }
-
 
 // Codes in the prefill GEMM's tiled layout (launch_prefill_prep): one block of 4 waves per tile as k_decode_split,
 // but each lane runs the two 32-symbol chains of its 64-symbol segment (split starts 2k and 2k + 1) interleaved, and
@@ -65,11 +64,12 @@ template <int SYMB>
 __global__ void __launch_bounds__(256) k_prefill_prep(DevMat M, uint8_t* __restrict__ out, int tr0, int tr1,
                                                       int stage_rows, PrefillX px) {
   typedef __attribute__((address_space(3))) const uint32_t LdsU32;
-  __shared__ __align__(16) uint32_t lut4[LUTN];  // the only static LDS object: at LDS address 0 (table_addr ORs it in)
+  // the only static LDS object, so at LDS address 0 (table_addr ORs its base in); an activation block's sums lie in it too
+  __shared__ __align__(16) uint32_t lut4[LUTN];
   extern __shared__ __align__(16) uint32_t tw[];
   const int KT = M.KT, KC = M.K / 32;
   if ((int)blockIdx.x < px.blocks) {
-    prefill_x_block(px, (int)blockIdx.x);
+    prefill_x_block(px, (int)blockIdx.x, reinterpret_cast<float*>(lut4));
     return;
   }
   const int t = tr0 * KT + (int)blockIdx.x - px.blocks;
@@ -162,7 +162,10 @@ bool decode_tiled_ok(const DevMat& M) {
 size_t prefill_x_bytes(int m, int K) { return (size_t)((m + 63) / 64 * 64) * K * 4; }
 size_t prefill_sx_bytes(int m, int K) { return (size_t)((m + 63) / 64 * 64) * (K / 32) * 4; }
 
-__global__ void __launch_bounds__(256) k_prefill_x(PrefillX px) { prefill_x_block(px, (int)blockIdx.x); }
+__global__ void __launch_bounds__(256) k_prefill_x(PrefillX px) {
+  __shared__ float part[PREFILL_X_LDS];
+  prefill_x_block(px, (int)blockIdx.x, part);
+}
 
 hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, const PrefillX* x, hipStream_t s) {
   if (!decode_tiled_ok(M) || tr0 < 0 || tr0 >= tr1 || tr1 > M.NT) return hipErrorInvalidValue;

@@ -76,7 +76,7 @@ def test_mfma_write_of_the_dpp_source_needs_the_matrix_core_wait():
 
 @pytest.fixture(scope="module")
 def kernels(lib, tmp_path_factory):
-    """The built library's gfx950 code objects: a function (symbol pattern) -> {mangled name: (object path)}."""
+    """The built library's gfx950 code objects: a function (symbol pattern) -> {mangled name: object path}."""
     d = tmp_path_factory.mktemp("objs")
     shutil.copy(_lib.LIB_PATH, d / "l.so")
     subprocess.run([OBJDUMP, "--offloading", "l.so"], cwd=d, check=True, stdout=subprocess.DEVNULL)
@@ -105,3 +105,18 @@ def test_wide_kernel_counts_a_row_after_every_waves_stores(kernels):
         after_store = before[max(i for i, op in enumerate(before) if op.startswith("global_store")) + 1:]
         wait = next((i for i, op in enumerate(after_store) if "vmcnt(0)" in op), None)
         assert wait is not None and "s_barrier" in after_store[wait:], name
+
+
+def test_kernels_with_their_table_at_lds_address_0_have_no_other_static_lds(kernels):
+    """The decode table of k_prefill_prep (2048 words, its base ORed into the index bits) and of k_fused_wide (indexed from
+    address 0, and 4 words after it) must be the kernel's only static LDS, since only then its place is known."""
+    for pattern, size in (("k_prefill_prep", 4 * 2048), ("k_fused_wide", 4 * (2048 + 4))):
+        found = kernels(pattern)
+        assert found
+        for name, obj in found.items():
+            notes = subprocess.run([os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf"), "--notes", obj], check=True,
+                                   text=True, stdout=subprocess.PIPE).stdout
+            fixed = [int(m.group(1)) for m in
+                     re.finditer(r"\.group_segment_fixed_size: (\d+)(?:(?!group_segment_fixed_size).)*?\.name:\s+%s\n" % name,
+                                 notes, re.S)]
+            assert fixed == [size], name
