@@ -103,9 +103,9 @@ int lw_group_matmul_dev(void* h, int count, const char* const* names, const void
  * buffered half-tile units per wave, the next one's copy in flight while one decodes) where the whole-tile kernel's
  * blocks would have fewer than 10 waves (few tiles per CU); m = 1 with int8 activations, the whole-tile kernel;
  * 2 <= m <= 4 with fp16 and 2 <= m <= 8 with int8 activations, every format, the whole-tile kernel with its products on
- * the matrix cores; 5 <= m <= 16 with fp16 and m <= 8 with fp32 activations (lw_matmul_dev, lw_matmul_dev_noalloc), every
- * format, the 16-token kernel (half a tile per wave, 16 rows x 16 tokens per matrix-core product, one launch per grouped
- * call after one that reorders the activations); otherwise the ring-staged kernels wherever a matrix has a ring
+ * the matrix cores; 5 <= m <= 16 with fp16 and m <= 8 with fp32 activations, every format, the 16-token kernel (half a tile
+ * per wave, 16 rows x 16 tokens per matrix-core product, one launch per grouped call after one that reorders the
+ * activations; packed matrices with fp32 activations and from 9 fp16 tokens); otherwise the ring-staged kernels wherever a matrix has a ring
  * schedule (the block-per-column kernel). 1 = the whole-tile fallback kernel everywhere; 2 = the block-per-column ring
  * kernel for every m; 7 = the ring-staged kernels for every m (for m = 1 the flat, load-balanced ring kernel);
  * 3 = as 7, but exception tiles are never decoded inside the flat launch (always by the separate exception pass);

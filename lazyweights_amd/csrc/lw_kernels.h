@@ -160,7 +160,7 @@ hipError_t launch_fused_tiles_mma8(const FlatPlan& plan, int per, hipStream_t s)
 int tiles_mma_max_waves(int kqt, int mt);  // the block limit of both matrix-core whole-tile kernels
 
 // The 16-token kernel (lw_wide.hip): mt <= 16 pseudo-tokens of fp16 activations (per = 2: fp32 activations as hi + lo
-// rows, mt / 2 tokens out), any mix of formats, blocks of W waves with half a tile each. Entry i owns wide_blocks(M, w)
+// rows, mt / 2 tokens out), any mix of formats (all coded or all packed), blocks of W waves with half a tile each. Entry i owns wide_blocks(M, w)
 // blocks from block0, at most w units (half tiles) each; w a multiple of 4 unless KT <= w, so that a matrix's results do
 // not depend on it. X: launch_wide_x's output. Y rows ldy apart; P: KT mt N partial slots (kNoPartial outside a launch),
 // cnt: 2 NT zeroed counters (left zeroed).

@@ -676,12 +676,16 @@ int halves_width(const lw::FlatPlan& fp, int mintiles, int& per) {
   return std::min(wmax, 2 * per);
 }
 
-// Whether the 16-token kernel takes a matrix (wide_ok) for mt pseudo-tokens in kernel mode 0: by the tokens alone, so
+// Whether the 16-token kernel takes a matrix for mt pseudo-tokens in kernel mode 0: by the tokens alone, so
 // that a matrix gives the same bits in a group and on its own. For 2..4 fp16 tokens k_fused_tiles_mma stays: us per call
 // against this kernel, Q4_K gate + up 29.3 / 29.5 at 2 tokens, 31.0 / 29.4 at 4, 31.6 / 29.2 at 5, 36.2 / 29.4 at 8, a
 // whole layer 43.5 / 46, 47.5 / 46, 52.5 / 46.3, 59.6 / 47; Q5_K gate + up 38.2 / 44.2 at 2, 44.0 / 44.2 at 5 (its waves
 // take tile after tile, so many tiles per CU cost it one start; with few per CU this kernel is ahead at 2 as well).
-bool wide_takes(int mt, int per) { return g_kernel_mode == 0 && mt <= 16 && (per == 2 ? mt >= 2 : mt >= 5); }
+// A packed matrix takes it with fp32 x and from 9 fp16 tokens, which keeps a twin at the coded matrix's bits there; up to 8
+// fp16 tokens it has those of the ring kernels (kernel mode 7).
+bool wide_takes(const lw::DevMat& dm, int mt, int per) {
+  return g_kernel_mode == 0 && mt <= 16 && (per == 2 ? mt >= 2 : mt >= (dm.packed ? 9 : 5)) && lw::wide_ok(dm);
+}
 
 // Its blocks (a wave per half tile; sets the entries' w and block0 and the plan's W): rows of at most 8 units whole, so
 // that a row's sum stays in the block (us per call at 5 tokens, rows of 8: q, k and v 13.3 with 8 waves, 15.0 with 4),
@@ -711,8 +715,7 @@ void wide_blocking(lw::WidePlan& wp) {
 }
 
 // Fused GEMV / skinny GEMM of `count` matrices with fp16 activations X[i] ([m * per][K_i] pseudo-tokens; x_f32, one
-// matrix, per = 2: fp32 [m][K], split into fp16 hi + lo on the device; twin: by the kernels that give a packed twin the
-// same bits):
+// matrix, per = 2: fp32 [m][K], split into fp16 hi + lo on the device):
 // ring-capable matrices go into grouped launches (same K-quant type and ring size, up to MAX_GROUP per launch), the
 // others into whole-tile launches. The ordered reduction over tile columns runs inside the flat (m = 1) launch for
 // every matrix that launch decodes completely, else in one reduction launch per MAX_GROUP matrices. Partials of
@@ -721,7 +724,7 @@ void wide_blocking(lw::WidePlan& wp) {
 // kernel modes 0, 3-5 and no packed matrix): int8 activations (quant_x8_dev) instead of X16.
 int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X, int count, int m, int per, float* const* Y,
                     const int* ldy, hipStream_t s, int* launches = nullptr, const X8* x8 = nullptr,
-                    const FixedScratch* fixed = nullptr, bool x_f32 = false, bool twin = false) {
+                    const FixedScratch* fixed = nullptr, bool x_f32 = false) {
   const int mt = m * per;
   std::vector<size_t> off(count + 1, 0);
   for (int i = 0; i < count; ++i) off[i + 1] = off[i] + (size_t)ts[i]->dm.KT * mt * ts[i]->N;
@@ -735,7 +738,6 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X, int count
     return dm.kqt >= lw::KQ_Q4_K && dm.kqt <= lw::KQ_IQ4_XS && !dm.packed && dm.dsplit && dm.lut4 && dm.rows &&
            dm.max_rows + 2 <= 256;
   };
-  const bool wide = !x8 && !twin && wide_takes(mt, per);
   const bool mma = !x8 && per == 1 && mt >= 2 && mt <= 4 && g_kernel_mode == 0;
   // its launches: matrices of one K-quant type, or of two (entries of the smaller type code first: one launch fewer),
   // up to MAX_GROUP each
@@ -876,16 +878,16 @@ int fused_group_dev(Model& M, Tensor* const* ts, const void* const* X, int count
   std::vector<lw::FlatPlan> flat_plans, split_plans;
   std::vector<std::pair<lw::FlatPlan, int>> tile_plans;  // whole-tile kernel launches and their tiles per block
   std::vector<std::pair<lw::FlatPlan, int>> half_plans;  // half-tile kernel launches and their tiles per block
-  // the 16-token whole-tile kernel over up to MAX_GROUP matrices of any formats, every tile and the reduction in the
-  // launch; the activations reordered first, each vector of the call once per symbol width
-  while (wide) {
+  // the 16-token kernel over up to MAX_GROUP matrices of any formats (coded or packed), every tile and the reduction in
+  // the launch; the activations reordered first, each vector of the call once per symbol width
+  while (!x8) {
     lw::WidePlan wp{};
     lw::WideXJobs xj{};
     std::vector<int> sel, job;
     size_t xbytes[lw::MAX_GROUP] = {}, xtotal = 0;
     for (int j = 0; j < count && wp.n < lw::MAX_GROUP; ++j) {
       const lw::DevMat& dm = ts[j]->dm;
-      if (done[j] || !lw::wide_ok(dm)) continue;
+      if (done[j] || !wide_takes(dm, mt, per) || (wp.n && dm.packed != wp.e[0].M.packed)) continue;
       int k = 0;
       while (k < xj.n && !(xj.X[k] == X[j] && xj.K[k] == dm.K && xj.symbits[k] == dm.symbits)) ++k;
       if (k == xj.n) {
@@ -1684,58 +1686,27 @@ int rt_test_matmul(void* h, const char* name, const float* X, int m, float* Y, i
   if (check_matmul(t, name)) return -1;
   const size_t K = (size_t)t->K, N = (size_t)t->N;
   float *dx = nullptr, *dy = nullptr;
-  void* dx16 = nullptr;
-  int rc = 0;
   auto cleanup = [&]() {
     if (dx) (void)hipFree(dx);
     if (dy) (void)hipFree(dy);
-    if (dx16) (void)hipFree(dx16);
   };
   if (hipMalloc(reinterpret_cast<void**>(&dy), (size_t)m * N * 4) != hipSuccess) {
     cleanup();
     g_err = "rt_test_matmul: device allocation failed";
     return -1;
   }
-  if (g_act8 && m <= 8 && path != 2) {  // int8 activations quantized on the device from the fp32 x
-    if (hipMalloc(reinterpret_cast<void**>(&dx), (size_t)m * K * 4) != hipSuccess ||
-        hipMemcpy(dx, X, (size_t)m * K * 4, hipMemcpyHostToDevice) != hipSuccess) {
-      cleanup();
-      g_err = "rt_test_matmul: upload failed";
-      return -1;
-    }
-    const void* xp = dx;
-    float* yp = dy;
-    const int ld = (int)N;
-    rc = act8_tokens(*M, &t, &xp, 0, 1, m, &yp, &ld, M->stream, nullptr);
-  } else if (m <= 8 && path != 2) {
-    // fp32 activations as fp16 hi + lo pseudo-tokens (x = hi + lo to 2^-22 relative)
-    std::vector<uint16_t> x16((size_t)2 * m * K);
-    for (int j = 0; j < m; ++j)
-      for (size_t k = 0; k < K; ++k) {
-        const float x = X[(size_t)j * K + k];
-        const uint16_t hi = lw::f32_to_f16(x);
-        x16[(2 * j) * K + k] = hi;
-        x16[(2 * j + 1) * K + k] = lw::f32_to_f16(x - lw::f16_to_f32(hi));
-      }
-    if (hipMalloc(&dx16, x16.size() * 2) != hipSuccess ||
-        hipMemcpy(dx16, x16.data(), x16.size() * 2, hipMemcpyHostToDevice) != hipSuccess) {
-      cleanup();
-      g_err = "rt_test_matmul: upload failed";
-      return -1;
-    }
-    // (the entry compares a matrix with its packed twin: the kernels that give both the same bits)
-    const void* xp = dx16;
-    const int ld = (int)N;
-    rc = fused_group_dev(*M, &t, &xp, 1, m, 2, &dy, &ld, M->stream, nullptr, nullptr, nullptr, false, true);
-  } else {
-    if (hipMalloc(reinterpret_cast<void**>(&dx), (size_t)m * K * 4) != hipSuccess ||
-        hipMemcpy(dx, X, (size_t)m * K * 4, hipMemcpyHostToDevice) != hipSuccess) {
-      cleanup();
-      g_err = "rt_test_matmul: upload failed";
-      return -1;
-    }
-    rc = decode_gemm_dev(*M, *t, dx, m, dy, (int)N, M->stream);
+  if (hipMalloc(reinterpret_cast<void**>(&dx), (size_t)m * K * 4) != hipSuccess ||
+      hipMemcpy(dx, X, (size_t)m * K * 4, hipMemcpyHostToDevice) != hipSuccess) {
+    cleanup();
+    g_err = "rt_test_matmul: upload failed";
+    return -1;
   }
+  const void* xp = dx;
+  const int ld = (int)N;
+  int rc;
+  if (m > 8 || path == 2) rc = decode_gemm_dev(*M, *t, dx, m, dy, ld, M->stream);
+  else if (g_act8) rc = act8_tokens(*M, &t, &xp, 0, 1, m, &dy, &ld, M->stream, nullptr);
+  else rc = fused_dev_f32(*M, *t, dx, m, dy, ld, M->stream);
   if (rc == 0) {
     if (hipStreamSynchronize(M->stream) != hipSuccess ||
         hipMemcpy(Y, dy, (size_t)m * N * 4, hipMemcpyDeviceToHost) != hipSuccess) {

@@ -61,8 +61,10 @@ constexpr int WIDE_MIN_ROWS = WIDE_TOKENS * 32 * 4 / 128;  // a buffer also hold
 
 __device__ __forceinline__ h2v dup(float v) { return h2v{(_Float16)v, (_Float16)v}; }
 
-// Half a tile (rows 32 f .. 32 f + 31) by one wave: chain c = 2 p + i is run 4 p + g of row 32 f + 16 i + j
-template <int KQ>
+// Half a tile (rows 32 f .. 32 f + 31) by one wave: chain c = 2 p + i is run 4 p + g of row 32 f + 16 i + j. PK: of a
+// packed matrix, each chain's 32 symbol bytes in registers and 256 table entries; the products, and so the results, are
+// those of the coded matrix with the same codes.
+template <int KQ, bool PK>
 struct WideUnit {
   static constexpr int SYMB = kq_symbits(KQ);
   static constexpr int TW = SYMB == 4 ? 2 * TK : TK;
@@ -77,6 +79,7 @@ struct WideUnit {
   static constexpr int NA = 2 * NSB;     // side records: a super-block of a row each (index 2 sb + i)
   // chain starts; side records as loaded (Q6_K: d and the scales of the run's sub-blocks of both passes)
   uint32_t start[4], raw[NA][5];
+  u32x4 sym[4][2];  // PK
   u32x4 x[XD][2], sx[NSB];
   __amdgpu_buffer_rsrc_t xr;
   uint32_t xv;  // the lane's 16 bytes of a piece (a lane past the tokens: past the buffer, reads zeros)
@@ -106,8 +109,15 @@ struct WideUnit {
       }
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      start[c] = M.hsplit[(((size_t)t * 2 + (uint32_t)f) * 64 + 32 * (c >> 1) + 16 * (c & 1)) * 4 + (uint32_t)(4 * j + g)];
+    for (int c = 0; c < 4; ++c) {
+      if constexpr (PK) {  // 16-byte pieces 2 r and 2 r + 1 of run r, [16 pieces][64 rows]
+        const u32x4* w = reinterpret_cast<const u32x4*>(M.words) + (size_t)t * 1024 + 512 * (c >> 1) + 32 * f + 16 * (c & 1);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sym[c][u] = w[128 * g + 64 * u + j];
+      } else {
+        start[c] = M.hsplit[(((size_t)t * 2 + (uint32_t)f) * 64 + 32 * (c >> 1) + 16 * (c & 1)) * 4 + (uint32_t)(4 * j + g)];
+      }
+    }
     const int xbytes = 2 * mt * K;
     xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(e->X), (short)0, xbytes + xbytes / 32 * 3, kBufferRsrcWord3);
     xv = j < mt ? (uint32_t)(16 * (g * mt + j)) : 0x7FFFFFF0u;
@@ -185,7 +195,7 @@ struct WideUnit {
     // P form: bit position in the buffer - GUARD_BITS + 64; slot = P >> 5 is the window row after the two in A and B
     uint32_t P[4], slot[4], A[4], B[4], C[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 4 && !PK; ++c) {
       P[c] = start[c] - (uint32_t)(32 * r0) - GUARD_BITS + 64u;
       slot[c] = __builtin_amdgcn_ubfe(P[c], 5, 8);
       const uint32_t a = rlb + (slot[c] << 7) + 64u * (c & 1);
@@ -214,24 +224,33 @@ struct WideUnit {
         }
       }
       uint32_t w1[4], e1[4], e2[4];
+      if constexpr (PK) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        w1[c] = __builtin_amdgcn_alignbit(B[c], A[c], P[c]);
-        e1[c] = *(LdsU32*)(w1[c] & 0x1FFCu);  // (the table lies at LDS address 0)
-      }
-      __builtin_amdgcn_sched_barrier(0);
+        for (int c = 0; c < 4; ++c) {
+          w1[c] = sym[c][q >> 3][q >> 1 & 3] >> (16 * (q & 1));
+          e1[c] = *(LdsU32*)(4u * (w1[c] & 255u));  // (the table lies at LDS address 0)
+          e2[c] = *(LdsU32*)(4u * (w1[c] >> 8 & 255u));
+        }
+      } else {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) e2[c] = *(LdsU32*)(w1[c] >> (e1[c] & 31u) & 0x1FFCu);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int c = 0; c < 4; ++c) {
+          w1[c] = __builtin_amdgcn_alignbit(B[c], A[c], P[c]);
+          e1[c] = *(LdsU32*)(w1[c] & 0x1FFCu);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        P[c] = P[c] + e1[c] + e2[c];
-        const uint32_t nslot = __builtin_amdgcn_ubfe(P[c], 5, 8);
-        const bool slide = nslot != slot[c];
-        A[c] = slide ? B[c] : A[c];
-        B[c] = slide ? C[c] : B[c];
-        slot[c] = nslot;
-        C[c] = *(LdsU32*)(rlb + (nslot << 7) + 64u * (c & 1));
+        for (int c = 0; c < 4; ++c) e2[c] = *(LdsU32*)(w1[c] >> (e1[c] & 31u) & 0x1FFCu);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          P[c] = P[c] + e1[c] + e2[c];
+          const uint32_t nslot = __builtin_amdgcn_ubfe(P[c], 5, 8);
+          const bool slide = nslot != slot[c];
+          A[c] = slide ? B[c] : A[c];
+          B[c] = slide ? C[c] : B[c];
+          slot[c] = nslot;
+          C[c] = *(LdsU32*)(rlb + (nslot << 7) + 64u * (c & 1));
+        }
       }
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
@@ -279,8 +298,8 @@ struct WideTag {
 
 }  // namespace
 
-// KQ: the entries' K-quant type, 0 for a plan over several
-template <int KQ>
+// KQ: the entries' K-quant type, 0 for a plan over several; PK: packed matrices
+template <int KQ, bool PK>
 __global__ void __launch_bounds__(64 * WIDE_MAX_WAVES) __attribute__((amdgpu_waves_per_eu(KQ == KQ_Q5_K || KQ == KQ_Q6_K ? 5 : 4)))
 k_fused_wide(WidePlan plan, int buf_rows) {
   __shared__ uint32_t lut4[LUTN + 4];  // the table first: table_addr takes it to lie at LDS address 0
@@ -316,11 +335,13 @@ k_fused_wide(WidePlan plan, int buf_rows) {
   if (threadIdx.x == 0) *last = 0u;
   f4v tot[2];
   auto run = [&](auto kq) __attribute__((always_inline)) {
-    WideUnit<decltype(kq)::value> unit;
+    WideUnit<decltype(kq)::value, PK> unit;
     const int sg = np > 1 ? 0 : wave / KT, hr = hr0 + sg, f = hr & 1, t = (hr >> 1) * KT + c0 + wave - sg * KT;
     int r0 = 0, nc = 0;
     if (have) {
       unit.load(e, t, f, mt, lane);
+    }
+    if (!PK && have) {
       // the unit's word rows (8 per instruction, the last masked)
       const uint32_t h = ((KU32*)e->M.hrow)[t];
       const uint32_t rw = ((KU32*)e->M.rows)[t >> 1] >> (16 * (t & 1)) & 0xFFFFu;
@@ -334,7 +355,7 @@ k_fused_wide(WidePlan plan, int buf_rows) {
     }
     {  // the decode table: 1 KB direct-to-LDS loads, chunk c by wave c mod W
       const uint4* ta = reinterpret_cast<const uint4*>(e->M.lut4);
-      for (int c = wave; c < 8; c += W)
+      for (int c = wave; c < (PK ? 1 : 8); c += W)
         __builtin_amdgcn_global_load_lds(ta + 64 * c + lane, (__attribute__((address_space(3))) void*)(lut4 + 256 * c), 16,
                                          0, 0);
     }
@@ -487,8 +508,8 @@ hipError_t launch_wide_x(WideXJobs q, hipStream_t s) {
 }
 
 bool wide_ok(const DevMat& M) {
-  return M.kqt >= KQ_Q4_K && M.kqt <= KQ_IQ4_XS && !M.packed && M.hsplit && M.lut4 && M.rows && M.tbase && M.side &&
-         M.hrow && M.max_rows + 2 <= 256;
+  return M.kqt >= KQ_Q4_K && M.kqt <= KQ_IQ4_XS && M.words && M.lut4 && M.side &&
+         (M.packed || (M.hsplit && M.rows && M.tbase && M.hrow && M.max_rows + 2 <= 256));
 }
 
 int wide_buf_rows(const WidePlan& p) {
@@ -506,7 +527,7 @@ hipError_t launch_fused_wide(const WidePlan& p, hipStream_t s) {
   int blocks = 0, kqt = p.e[0].M.kqt;
   for (int i = 0; i < p.n; ++i) {
     const WideEntry& e = p.e[i];
-    if (!wide_ok(e.M) || !e.X || ((uintptr_t)e.X & 15) || !e.Y || !e.P || !e.cnt || e.block0 != blocks || e.M.KT < 1 ||
+    if (!wide_ok(e.M) || e.M.packed != p.e[0].M.packed || !e.X || ((uintptr_t)e.X & 15) || !e.Y || !e.P || !e.cnt || e.block0 != blocks || e.M.KT < 1 ||
         e.M.NT < 1 || e.w < 1 || (e.M.KT <= e.w ? e.w / e.M.KT * e.M.KT : e.w) > p.W || (e.M.KT > e.w && e.w % 4))
       return hipErrorInvalidValue;
     blocks += wide_blocks(e.M, e.w);
@@ -515,9 +536,10 @@ hipError_t launch_fused_wide(const WidePlan& p, hipStream_t s) {
   const int rows = wide_buf_rows(p);
   if (wide_lds_bytes(p.W, rows) > 160 * 1024) return hipErrorInvalidValue;
   const size_t smem = (size_t)p.W * rows * 128;
-  auto* const kernel = kqt == KQ_Q4_K ? k_fused_wide<KQ_Q4_K> : kqt == KQ_Q5_K ? k_fused_wide<KQ_Q5_K>
-                     : kqt == KQ_Q6_K ? k_fused_wide<KQ_Q6_K> : kqt == KQ_IQ4_XS ? k_fused_wide<KQ_IQ4_XS>
-                                                              : k_fused_wide<0>;
+  auto* const kernel = p.e[0].M.packed ? k_fused_wide<0, true>
+                     : kqt == KQ_Q4_K ? k_fused_wide<KQ_Q4_K, false> : kqt == KQ_Q5_K ? k_fused_wide<KQ_Q5_K, false>
+                     : kqt == KQ_Q6_K ? k_fused_wide<KQ_Q6_K, false> : kqt == KQ_IQ4_XS ? k_fused_wide<KQ_IQ4_XS, false>
+                                                                     : k_fused_wide<0, false>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return e;

@@ -1,6 +1,7 @@
 """The 16-token half-tile kernel (lw_wide.hip) through the C-ABI, against fp64: every format, the smallest shapes and the
 ones that put a row of units into one block, across two and across many, 5..16 tokens of fp16 and 1..8 of fp32
-activations, groups of several formats in one call, activations at any alignment, and a caller's scratch at its limit."""
+activations, groups of several formats in one call, activations at any alignment, a caller's scratch at its limit, large
+activations and packed twins."""
 import ctypes
 
 import numpy as np
@@ -140,3 +141,41 @@ def test_sub_block_sums_past_fp16(gpu, lib, orc, tmp_path, kqt):
             assert e.max() < TOL, (m, f16)
     finally:
         rt.close()
+
+
+@pytest.mark.parametrize("kqt", (1, 2, 3, 4))
+def test_packed_twin_and_host_entry(gpu, lib, orc, tmp_path, kqt):
+    """A packed twin gives the coded matrix's bits with fp32 activations and with 9..16 tokens of fp16 (row units: 1, 8 in one
+    block, 9 over several), alone and grouped over two formats; rt_test_matmul gives lw_matmul_dev's."""
+    import torch
+    from lazyweights_amd import Runtime, bundle
+    cols = 512 if kqt in (1, 4) else 256
+    mats = [("r%d" % i, kqt, n, k * cols, H[kqt], 950 + i) for i, (n, k) in enumerate(((64, 1), (192, 8), (128, 9)))]
+    mats.append(("o", kqt % 4 + 1, 64, 9 * 512, H[kqt % 4 + 1], 960))
+    bundle.write_synthetic_bundle(str(tmp_path / "coded"), mats, threads=16)
+    bundle.write_packed_bundle(str(tmp_path / "packed"), mats, threads=16)
+    with Runtime(tmp_path / "coded") as rc, Runtime(tmp_path / "packed") as rp:
+        for name, kq, N, K, _, seed in mats:
+            w = bundle.synth_matrix(kq, N, K, H[kq], seed, threads=16)
+            for m, f16 in ((1, False), (3, False), (8, False), (9, True), (16, True)):
+                x = torch.randn(m, K, generator=torch.Generator().manual_seed(seed + m))
+                x = (x.half() if f16 else x).cuda()
+                yc, yp = (torch.full((m, N), float("nan"), device="cuda") for _ in range(2))
+                rc.matmul_dev(name, x, yc, x_f16=f16)
+                for _ in range(2):
+                    rp.matmul_dev(name, x, yp, x_f16=f16)
+                torch.cuda.synchronize()
+                assert torch.equal(yc, yp), (name, m, f16)
+                assert err(yp, y64(orc, kq, w, x)) < TOL, (name, m, f16)
+                if not f16:
+                    for rt in (rc, rp):
+                        assert np.array_equal(rt.test_matmul(name, x.cpu().numpy()), yc.cpu().numpy()), (name, m)
+        n, xs = len(mats), [torch.randn(11, m[3], generator=torch.Generator().manual_seed(m[3])).half().cuda() for m in mats]
+        ys = []
+        for rt in (rc, rp):
+            ys.append([torch.zeros(11, m[2], device="cuda") for m in mats])
+            assert lib.lw_group_matmul_dev(rt.h, n, (ctypes.c_char_p * n)(*[m[0].encode() for m in mats]),
+                                           (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs]), 11,
+                                           (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys[-1]]), None) == 0
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(*ys))
