@@ -21,9 +21,10 @@
 // Weights. A product's weights lie in 4 sub-blocks (the runs g), so they are scaled by their sub-blocks' integer scales
 // before it, exactly in fp16:
 //   Q4_K: sc q 2^-24 from the table's grid byte as a denormal, Q5_K: sc q (at most 63 x 31);
-//   Q6_K, IQ4_XS: s f(q) has up to 13 bits, so s = s1 + s0 with s1 even and s0 its low bit: s1 f(q) (even, at most 4096)
-//   and s0 f(q) are exact and both products go to one accumulator; IQ4_XS's kv / 16 = fp16(64 + b / 16) - 72 of the grid
-//   byte b = kv + 128, one fma per product.
+//   Q6_K, IQ4_XS: s f(q) has up to 13 bits, so s = s1 + s0 with s1 even and s0 = 1 or 2 of its sign (split_scale): s1 f(q)
+//   and s0 f(q) are exact and both products go to one accumulator. Neither part is 0 unless s is, nor do their signs
+//   differ, so an infinite activation stays infinite; IQ4_XS's kv / 16 = fp16(64 + b / 16) - 72 of the grid byte
+//   b = kv + 128, one fma per product.
 // d is applied in fp32 when the super-block is complete. Mins (Q4_K / Q5_K): one product per row group and super-block of
 // the mins with the sub-blocks' fp32 x sums, formed by launch_wide_x and held as three bf16 parts that add up to all 24
 // bits (as fp16 hi and lo a sum past 65504, 32 activations of 2047, would be infinite): parts in lane groups 0, 1 and 2 of
@@ -60,6 +61,12 @@ constexpr int WIDE_TOKENS = 16;
 constexpr int WIDE_MIN_ROWS = WIDE_TOKENS * 32 * 4 / 128;  // a buffer also holds its unit's results
 
 __device__ __forceinline__ h2v dup(float v) { return h2v{(_Float16)v, (_Float16)v}; }
+
+// s0 of a scale v in -128 .. 127: 1 or 2 with v's sign so that v - s0 is even, half of v up to 2
+__device__ __forceinline__ float split_scale(int v) {
+  const float f = (float)v, part = __builtin_copysignf((float)(2 - (v & 1)), f);
+  return __builtin_fabsf(f) <= 2.f ? 0.5f * f : part;
+}
 
 // Half a tile (rows 32 f .. 32 f + 31) by one wave: chain c = 2 p + i is run 4 p + g of row 32 f + 16 i + j. PK: of a
 // packed matrix, each chain's 32 symbol bytes in registers and 256 table entries; the products, and so the results, are
@@ -203,7 +210,7 @@ struct WideUnit {
       B[c] = *(LdsU32*)(a - 128u);
       C[c] = *(LdsU32*)a;
     }
-    h2v s1[4], n1[4], s0[4], n0[4];  // the chains' current scales (SPLIT: s1 even + s0) and IQ4_XS's -72 s
+    h2v s1[4], n1[4], s0[4], n0[4];  // the chains' current scales (SPLIT: s1 + s0) and IQ4_XS's -72 s
     uint32_t w4[4][2];
     static_for<16>([&](auto pc) {
       constexpr int q = decltype(pc)::value, st = q / PPS;
@@ -216,10 +223,11 @@ struct WideUnit {
             s1[c] = dup((float)b);
           } else {
             const int v = KQ == KQ_Q6_K ? (int)(int8_t)(uint8_t)b : (int)b - 32;
-            s1[c] = dup((float)(v & ~1));
-            s0[c] = dup((float)(v & 1));
-            n1[c] = dup(-72.f * (float)(v & ~1));
-            n0[c] = dup(-72.f * (float)(v & 1));
+            const float b0 = split_scale(v), b1 = (float)v - b0;
+            s1[c] = dup(b1);
+            s0[c] = dup(b0);
+            n1[c] = dup(-72.f * b1);
+            n0[c] = dup(-72.f * b0);
           }
         }
       }

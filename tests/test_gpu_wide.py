@@ -1,7 +1,7 @@
 """The 16-token half-tile kernel (lw_wide.hip) through the C-ABI, against fp64: every format, the smallest shapes and the
 ones that put a row of units into one block, across two and across many, 5..16 tokens of fp16 and 1..8 of fp32
 activations, groups of several formats in one call, activations at any alignment, a caller's scratch at its limit, large
-activations and packed twins."""
+and infinite activations and packed twins."""
 import ctypes
 
 import numpy as np
@@ -179,3 +179,30 @@ def test_packed_twin_and_host_entry(gpu, lib, orc, tmp_path, kqt):
                                            (ctypes.c_void_p * n)(*[y.data_ptr() for y in ys[-1]]), None) == 0
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(*ys))
+
+
+@pytest.mark.parametrize("kqt", (3, 4))
+def test_infinite_activation(gpu, lib, orc, tmp_path, kqt):
+    """An infinite fp16 activation gives infinities of its products' signs in Q6_K and IQ4_XS, which have no mins (and NaN
+    where the weight is 0), and leaves the other tokens alone."""
+    import torch
+    rt, w = open_mats(tmp_path, [("a", kqt, 128, 4608, H[kqt], 33)])
+    try:
+        d = orc.dequant(kqt, *w["a"])
+        for m in (5, 9, 16):
+            x = torch.randn(m, 4608, generator=torch.Generator().manual_seed(m)).half()
+            x[1, 700], x[m - 1, 4000] = float("inf"), float("-inf")
+            y = torch.zeros(m, 128, device="cuda")
+            xd = x.cuda()
+            assert lib.lw_matmul_dev(rt.h, b"a", xd.data_ptr(), 1, m, y.data_ptr(), 128, None) == 0
+            torch.cuda.synchronize()
+            y = y.cpu().numpy()
+            with np.errstate(invalid="ignore"):
+                for tok, col, sign in ((1, 700, 1), (m - 1, 4000, -1)):
+                    want = sign * np.inf * d[:, col]
+                    print("inf", kqt, m, int(np.isinf(y[tok]).sum()), "of", int(np.isinf(want).sum()), flush=True)
+                    assert np.array_equal(y[tok], want, equal_nan=True), (m, tok)
+            keep = [t for t in range(m) if t not in (1, m - 1)]
+            assert err(torch.from_numpy(y[keep]), y64(orc, kqt, w["a"], x[keep])) < TOL
+    finally:
+        rt.close()
