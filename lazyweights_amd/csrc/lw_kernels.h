@@ -244,7 +244,11 @@ hipError_t launch_decode_hilo(const DevMat& M, int tr0, int tr1, void* WW, hipSt
 // (launch_prefill_prep) and x in its tiled layouts (SXT read for Q4_K / Q5_K only); K a multiple
 // of 256
 hipError_t launch_gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int nrows, const void* XT,
-                               const void* SXT, int m, float* Y, int ldy, hipStream_t s);
+                               const void* SXT, int m, int tiles, float* Y, int ldy, hipStream_t s);
+// its tiles (weight rows x tokens per wave) and waves per block, for a matrix of `rows` tile rows taken at most `chunk` at a
+// time
+enum : int { PREFILL_64X64_4, PREFILL_64X64_8, PREFILL_64X32_4, PREFILL_64X32_8 };
+int prefill_tiles(int rows, int chunk, int m);
 // Codes of tile rows [tr0, tr1) in the prefill GEMM's tiled layout: per 32-row tile and 32-code chunk a 1 KB piece,
 // lane (h, c) = 32 h + c holding row c's codes 16 h .. 16 h + 15 of the chunk (IQ4_XS: their grid bytes kv[q] + 128);
 // needs decode_tiled_ok (packed matrices, coded ones with split offsets). With x in the same launch: fp32 X [m][K] -> XT

@@ -1,4 +1,6 @@
 // Prefill (m > 8): codes decoded to a tiled layout, activations split and tiled, GEMM on the matrix cores.
+#include <algorithm>
+
 #include "lw_device.h"
 
 namespace lw {
@@ -661,32 +663,50 @@ static hipError_t gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int
   return hipGetLastError();
 }
 
+// 64 x 64 or 64 x 32 tiles (rows x tokens) per wave, for a matrix of `rows` row pairs whose GEMM runs over at most `chunk` of
+// them at a time (both of the matrix alone, not of what the scratch has grown to: the same bits from call to call). A larger
+// tile takes 3/4 of the time per product, but its blocks fill the 256 CUs in coarser steps and may hold 32 tokens of
+// padding. Time goes with the fullest CU's blocks and, a quarter as much, with all of them: c(b) = 3 ceil(b / 256) + b / 256
+// per launch. Fitted to 230 shapes of all formats (m = 9 .. 2048, N = 2048 .. 28672, K = 512 .. 14336): within 1 % of the best
+// of the four on the mean. us per call, preparation included, of 64 x 64 by 4 waves / by 8 / 64 x 32 by 4 / by 8: Q4_K
+// 14336 x 4096, m = 9 36.6 / 34.0 / 32.9 / 30.1, m = 33 36.5 / 34.0 / 39.2 / 42.4, m = 2048 546 / 580 / 674 / 736; Q6_K
+// 16384 x 1024, m = 65 29.0 / 30.5 / 24.4 / 27.4; IQ4_XS 6400 x 14336 (two launches), m = 200 192 / 190 / 157 / 157, m = 300
+// 204 / 204 / 226 / 231; Q4_K 2048 x 14336, m = 300 75 / 68 / 78 / 82.
+// K split over 4 waves where the blocks are more than the CUs, else over 8.
+int prefill_tiles(int rows, int chunk, int m) {
+  long long c64 = 0, c32 = 0;
+  const long long t64 = (m + 63) / 64, t32 = (m + 31) / 32, first = std::min(rows, chunk);
+  for (long long r = rows; r > 0; r -= chunk) {
+    const long long n = std::min<long long>(r, chunk), b64 = n * t64, b32 = n * t32;
+    c64 += (b64 + 255) / 256 * 768 + b64;
+    c32 += (b32 + 255) / 256 * 768 + b32;
+  }
+  if (2 * c32 > 3 * c64) return first * t64 > 256 ? PREFILL_64X64_4 : PREFILL_64X64_8;
+  return first * t32 > 256 ? PREFILL_64X32_4 : PREFILL_64X32_8;
+}
+
 template <int KQ>
 static hipError_t gemm_prefill_any(const DevMat& M, const uint8_t* CT, int row0, int nrows, const uint16_t* x,
-                                   const uint16_t* sx, int m, float* Y, int ldy, hipStream_t s) {
-  // 64 x 64 tiles per wave where they make 192 blocks (3/4 of the CUs), else 64 x 32; the K split over 4 waves where the
-  // blocks are more than the CUs, else over 8: us per call (preparation included) with 64 x 64 by 4 waves / by 8 / 64 x 32
-  // by 4 / by 8: Q4_K 14336 x 4096, m = 64 (224 blocks of 64 x 64) 38.6 / 37.9 / 41.2 / 45.7, m = 128 53 / 56 / 61 / 70,
-  // m = 2048 528 / 581 / 651 / 728; 4096 x 4096, m = 128 (128) 27.5 / 26.4 / 22.0 / 23.1, m = 512 (512) 46 / 48 / 50 / 61;
-  // 1024 x 4096, m = 128 (32) 25.1 / 23.8 / 19.0 / 18.3; Q6_K 4096 x 14336, m = 512 (512) 170 / 171 / 190 / 200. (By the
-  // matrix's rows, not the chunk's.)
-  const long long rows64 = M.N / 64, b64 = rows64 * ((m + 63) / 64), b32 = rows64 * ((m + 31) / 32);
-  if (b64 > 256) return gemm_prefill<KQ, 2, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-  if (b64 >= 192) return gemm_prefill<KQ, 2, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-  if (b32 >= 256) return gemm_prefill<KQ, 1, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-  return gemm_prefill<KQ, 1, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+                                   const uint16_t* sx, int m, int tiles, float* Y, int ldy, hipStream_t s) {
+  switch (tiles) {
+    case PREFILL_64X64_4: return gemm_prefill<KQ, 2, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case PREFILL_64X64_8: return gemm_prefill<KQ, 2, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case PREFILL_64X32_4: return gemm_prefill<KQ, 1, 4>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case PREFILL_64X32_8: return gemm_prefill<KQ, 1, 8>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_gemm_prefill(const DevMat& M, const uint8_t* CT, int row0, int nrows, const void* XT,
-                               const void* SXT, int m, float* Y, int ldy, hipStream_t s) {
+                               const void* SXT, int m, int tiles, float* Y, int ldy, hipStream_t s) {
   if (nrows < 1 || m < 1 || nrows % 64 || M.K % 256) return hipErrorInvalidValue;
   const uint16_t* x = static_cast<const uint16_t*>(XT);
   const uint16_t* sx = static_cast<const uint16_t*>(SXT);
   switch (M.kqt) {
-    case KQ_Q4_K: return gemm_prefill_any<KQ_Q4_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-    case KQ_Q5_K: return gemm_prefill_any<KQ_Q5_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-    case KQ_Q6_K: return gemm_prefill_any<KQ_Q6_K>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
-    case KQ_IQ4_XS: return gemm_prefill_any<KQ_IQ4_XS>(M, CT, row0, nrows, x, sx, m, Y, ldy, s);
+    case KQ_Q4_K: return gemm_prefill_any<KQ_Q4_K>(M, CT, row0, nrows, x, sx, m, tiles, Y, ldy, s);
+    case KQ_Q5_K: return gemm_prefill_any<KQ_Q5_K>(M, CT, row0, nrows, x, sx, m, tiles, Y, ldy, s);
+    case KQ_Q6_K: return gemm_prefill_any<KQ_Q6_K>(M, CT, row0, nrows, x, sx, m, tiles, Y, ldy, s);
+    case KQ_IQ4_XS: return gemm_prefill_any<KQ_IQ4_XS>(M, CT, row0, nrows, x, sx, m, tiles, Y, ldy, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -1423,11 +1423,12 @@ int decode_gemm_dev(Model& M, Tensor& t, const float* X, int m, float* Y, int ld
       return -1;
     const bool mins = t.kqt == lw::KQ_Q4_K || t.kqt == lw::KQ_Q5_K;
     const lw::PrefillX px{X, M.X16, mins ? M.SX : nullptr, m, (int)t.K, 0};
+    const int tiles = lw::prefill_tiles(t.dm.NT, (int)(cap / row_bytes), m);
     const int rows_fit = (int)std::max<size_t>(1, M.codes_cap / row_bytes);
     for (int tr0 = 0; tr0 < t.dm.NT; tr0 += rows_fit) {
       const int tr1 = std::min(t.dm.NT, tr0 + rows_fit);
       HIPCHECK(lw::launch_prefill_prep(t.dm, M.codes, tr0, tr1, tr0 ? nullptr : &px, s));
-      HIPCHECK(lw::launch_gemm_prefill(t.dm, M.codes, tr0 * lw::TN, (tr1 - tr0) * lw::TN, M.X16, M.SX, m, Y, ldy, s));
+      HIPCHECK(lw::launch_gemm_prefill(t.dm, M.codes, tr0 * lw::TN, (tr1 - tr0) * lw::TN, M.X16, M.SX, m, tiles, Y, ldy, s));
     }
     return 0;
   }

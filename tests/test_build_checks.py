@@ -1,6 +1,7 @@
 """The build's DPP wait-state check (lazyweights_amd/build.py dpp_violations) on hand-written disassembly: the
 hazards it must refuse and the forms it must accept (the check guards the inline-assembly DPP products, which the
-compiler's hazard recognizer does not see); and properties of the built kernels that no run shows reliably."""
+compiler's hazard recognizer does not see); properties of the built kernels that no run shows reliably; and the prefill GEMM's
+choice of tiles."""
 import os
 import re
 import shutil
@@ -120,3 +121,15 @@ def test_kernels_with_their_table_at_lds_address_0_have_no_other_static_lds(kern
                      re.finditer(r"\.group_segment_fixed_size: (\d+)(?:(?!group_segment_fixed_size).)*?\.name:\s+%s\n" % name,
                                  notes, re.S)]
             assert fixed == [size], name
+
+
+def test_prefill_tiles_of_calls_that_were_slower(lib):
+    """Tile rows, tile rows per launch and tokens where 64 x 64 tiles lose to 64 x 32 ones (64 rows x tokens per wave; by 4
+    and by 8 waves: 0 and 1, 2 and 3) by up to a quarter: few tokens of a 64-token tile, or a second block on few CUs; and
+    ones where they win."""
+    tiles = lib._ZN2lw13prefill_tilesEiii
+    for rows, chunk, m in ((224, 224, 9), (256, 256, 9), (256, 256, 65), (100, 73, 65), (100, 73, 200), (80, 73, 200)):
+        assert tiles(rows, chunk, m) >= 2, (rows, m)
+    for rows, chunk, m in ((224, 224, 33), (224, 224, 2048), (64, 64, 512), (100, 73, 300), (100, 73, 400), (32, 32, 300)):
+        assert tiles(rows, chunk, m) <= 1, (rows, m)
+    assert tiles(448, 448, 9) == 2 and tiles(16, 16, 128) == 3  # more blocks than CUs, fewer
