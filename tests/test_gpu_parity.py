@@ -947,9 +947,8 @@ def test_gpu_model_shaped_bundle(gpu, tmp_path, orc):
 
 @pytest.mark.parametrize("kqt,K", [(1, 1024), (2, 768), (3, 768), (4, 1024)])
 def test_gpu_prefill_tile_shapes(gpu, tmp_path, orc, kqt, K):
-    """The prefill GEMM's block shapes at their edges: 64 x 64 tiles by 4 waves (from 192 blocks: 192 x 64 rows and one
-    token tile pair, ragged token counts, three pairs), 64 x 32 tiles by 4 waves (from 256 blocks) and by 8 below, with
-    fewer super-blocks than waves. The tolerance is the fp32 sums' (2-norm), far below a wrong tile or scale."""
+    """The prefill GEMM with fewer super-blocks than waves (3 or 4), at ragged token counts: 64 x 32 tiles by 8 waves and by 4,
+    64 x 64 tiles by 8. The tolerance is the fp32 sums' (2-norm), far below a wrong tile or scale."""
     import torch
     from lazyweights_amd import Runtime, bundle
     mats = [("p%d" % N, kqt, N, K, {1: 2.3, 2: 3.4, 3: 4.3, 4: 2.6}[kqt], 700 + N) for N in (64, 4096, 12288)]
@@ -966,3 +965,27 @@ def test_gpu_prefill_tile_shapes(gpu, tmp_path, orc, kqt, K):
                 e = np.linalg.norm(y.double().cpu().numpy() - y64) / np.linalg.norm(y64)
                 say("prefill tiles", name, kqt, "m", m, "err %.2g" % e)
                 assert e < 1e-6
+
+
+@pytest.mark.parametrize("kqt,K", [(1, 2560), (2, 2304), (3, 2304), (4, 2560)])
+def test_gpu_prefill_block_shapes(gpu, lib, tmp_path, orc, kqt, K):
+    """Every block shape of the prefill GEMM with an odd number of row pairs, token tiles in several groups of 4 with a last
+    one of 1 (5 and 9 pairs), blocks not a multiple of 8, and 9 or 10 super-blocks, so that every one of 4 waves puts its
+    totals aside once and the waves' shares differ. y is NaN before the call. The tolerance is the fp32 sums' (2-norm)."""
+    import torch
+    from lazyweights_amd import Runtime, bundle
+    tiles = {(4288, 300): 0, (2368, 560): 0, (4288, 130): 1, (8320, 70): 2, (4288, 33): 3}
+    names = {N: ("b%d" % N, kqt, N, K, {1: 2.3, 2: 3.4, 3: 4.3, 4: 2.6}[kqt], 800 + N) for N, _ in tiles}
+    bundle.write_synthetic_bundle(str(tmp_path), list(names.values()), threads=16)
+    with Runtime(tmp_path) as rt:
+        for (N, m), want in tiles.items():
+            assert lib._ZN2lw13prefill_tilesEiii(N // 64, N // 64, m) == want
+            x = torch.randn(m, K, generator=torch.Generator().manual_seed(m))
+            y = torch.full((m, N), float("nan"), device="cuda")
+            rt.matmul_dev(names[N][0], x.cuda(), y, x_f16=False)
+            torch.cuda.synchronize()
+            w = orc.dequant(kqt, *bundle.synth_matrix(*names[N][1:], threads=16))
+            y64 = x.double().numpy() @ w.astype(np.float64).T
+            e = np.linalg.norm(y.double().cpu().numpy() - y64) / np.linalg.norm(y64)
+            say("prefill blocks", kqt, N, "m", m, "err %.2g" % e)
+            assert e < 1e-6
