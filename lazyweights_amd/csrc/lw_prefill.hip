@@ -209,9 +209,10 @@ hipError_t launch_prefill_prep(const DevMat& M, uint8_t* out, int tr0, int tr1, 
 // cycle of a CU where its vector cache gives 64; with TT = 2 the same codes serve 16 products (80 bytes a cycle, and half
 // the scaling of codes per product). 64 x 64 tiles take all 256 registers of 2 waves per SIMD (128 in accumulators): the
 // operand rings are 2 chunks deep instead of 4, side records and x sums are read through buffers (no per-lane addresses)
-// half a super-block ahead, and a tile's registers take its mins product once it is folded. Q4_K 14336 x 4096, m = 2048:
-// 728 -> 516 us with the preparation (526 with the totals put aside, below), 496 useful TFLOP/s in the GEMM = 992 of
-// products, where a library fp16 GEMM of 8192 x 8192 x 8192 reaches 1176 on this card.
+// two chunks ahead, and a tile's registers take its mins product before its own. Q4_K 14336 x 4096, m = 2048: 737 -> 520 us
+// with the preparation, the totals put aside (below) included: 462 useful TFLOP/s a call, two products per weight, where a
+// library fp16 GEMM of 8192 x 8192 x 8192 reaches 1176 on this card. Mins folded after the products instead: 527 us, 5
+// registers spilled, and 1.2 % further from 64 bits.
 // codes q0..q3 (bytes of qw) -> sc q / 16 as 4 fp16 in two words (nsc = -64 sc)
 __device__ __forceinline__ uint2 scaled_codes16(uint32_t qw, h2v sc, h2v nsc) {
   const h2v a = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(0x54545454u, qw, 0x04010400u));
@@ -397,15 +398,21 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
   f16x16 tot[2][TT] = {};
   extern __shared__ float part[];
   // with 4 waves sharing K the totals are put aside half way, as in k_gemm_prefill_sub: 14336 x 4096, m = 2048 1.8e-7
-  // from 64 bits without, 1.7e-7 with 8 waves and with this, which takes 512 -> 526 us (6 registers spill around it)
+  // from 64 bits without, 1.7e-7 with 8 waves and with this, for 1 to 2 % of the time
   int left = WV < 8 ? ((NB - wave + WV - 1) / WV + 1) / 2 : 0;
   bool aside = false;
   f4v* const own = reinterpret_cast<f4v*>(part) + wave * 2 * TT * 256 + lane;
   uint32_t swa[5] = {}, swb[5] = {};
   u32x4 qa[RD] = {}, qb[RD] = {}, xr[RD][4 * TT] = {};
+  u32x4 sx[TT] = {};  // Sx of the super-block: lanes h = 0 the hi, h = 1 the lo halves
+  auto load_sx = [&](int sb) {
+#pragma unroll
+    for (int b = 0; b < TT; ++b) sx[b] = __builtin_amdgcn_raw_buffer_load_b128(rsx, vo, (b * NB + sb) * 1024, 0);
+  };
   if (wave < NB) {
     side_fetch<KQ>(rs, vs, wave * (64 * SB), swa);
     side_fetch<KQ>(rs, vs + 32 * SB, wave * (64 * SB), swb);
+    load_sx(wave);
 #pragma unroll
     for (int i = 0; i < RD - 1; ++i) {
       load_q(wave * 8 + i, qa[i], qb[i]);
@@ -415,8 +422,26 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
   for (int sb = wave; sb < NB; sb += WV) {
     const KSide ka = kside(swa), kb = kside(swb);
     const int nsb = sb + WV;
-    u32x4 sx[TT];  // Sx of this super-block, loaded at chunk 5: lanes h = 0 the hi, h = 1 the lo halves
-    f16x16 d[2][TT] = {};
+    f16x16 d[2][TT];
+    // mins, into the totals before the super-block's products (which are the larger term): A2 = the tokens' Sx over the 8
+    // sub-blocks, hi in k 0..7 and lo in k 8..15, B2 = the row's 8 mins in both; in the tiles' registers
+    const h8v mn[2] = {kside_mins(ka), kside_mins(kb)};
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < TT; ++b)
+        d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sx[b]), mn[a], f16x16{}, 0, 0, 0);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      const float dmin = a ? kb.dmin : ka.dmin;
+#pragma unroll
+      for (int b = 0; b < TT; ++b) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(-dmin, d[a][b][r], tot[a][b][r]);
+        asm volatile("" : "+v"(tot[a][b]));
+        d[a][b] = f16x16{};
+      }
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {  // the super-block's 8 chunks (sub-blocks)
       if (j < 9 - RD || nsb < NB) {
@@ -424,13 +449,10 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
         load_q(kn, qa[(j + RD - 1) % RD], qb[(j + RD - 1) % RD]);
         load_x(kn, xr[(j + RD - 1) % RD]);
       }
-      if (j == 5) {
-#pragma unroll
-        for (int b = 0; b < TT; ++b) sx[b] = __builtin_amdgcn_raw_buffer_load_b128(rsx, vo, (b * NB + sb) * 1024, 0);
-      }
-      if (j == 5 && nsb < NB) {  // the next super-block's records (from the start they would cost 10 registers more)
+      if (j == 6 && nsb < NB) {  // the next super-block's records and sums (from chunk 5 on they would spill 8 registers)
         side_fetch<KQ>(rs, vs, nsb * (64 * SB), swa);
         side_fetch<KQ>(rs, vs + 32 * SB, nsb * (64 * SB), swb);
+        load_sx(nsb);
       }
       __builtin_amdgcn_sched_barrier(0);  // keep the loads issued here, ahead of this chunk's products
       const u32x4 ca = qa[j % RD], cb = qb[j % RD];
@@ -453,29 +475,13 @@ __global__ void __launch_bounds__(64 * WV, 2 * 4 / WV) k_gemm_prefill(DevMat M, 
               d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, xc[4 * b + 2 * half + st]), w[a], d[a][b], 0, 0, 0);
       }
     }
-    // mins: A2 = the tokens' Sx over the super-block's 8 sub-blocks, hi in k 0..7 and lo in k 8..15, B2 = the row's 8
-    // mins in both
-    const h8v mn[2] = {kside_mins(ka), kside_mins(kb)};
 #pragma unroll
     for (int a = 0; a < 2; ++a) {
       const float d16 = a ? kb.d16 : ka.d16;
 #pragma unroll
-      for (int b = 0; b < TT; ++b) {
-        // (the tile's registers take the mins product once they are folded)
+      for (int b = 0; b < TT; ++b)
 #pragma unroll
         for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(d16, d[a][b][r], tot[a][b][r]);
-        asm volatile("" : "+v"(tot[a][b]));
-        d[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, sx[b]), mn[a], f16x16{}, 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const float dmin = a ? kb.dmin : ka.dmin;
-#pragma unroll
-      for (int b = 0; b < TT; ++b) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tot[a][b][r] = fmaf(-dmin, d[a][b][r], tot[a][b][r]);
-      }
     }
     if (WV < 8 && --left == 0 && nsb < NB) {
       aside = true;

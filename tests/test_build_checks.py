@@ -133,3 +133,15 @@ def test_prefill_tiles_of_calls_that_were_slower(lib):
     for rows, chunk, m in ((224, 224, 33), (224, 224, 2048), (64, 64, 512), (100, 73, 300), (100, 73, 400), (32, 32, 300)):
         assert tiles(rows, chunk, m) <= 1, (rows, m)
     assert tiles(448, 448, 9) == 2 and tiles(16, 16, 128) == 3  # more blocks than CUs, fewer
+
+
+def test_prefill_gemm_keeps_its_tiles_in_registers(kernels):
+    """No form of the prefill GEMM spills: its 64 x 64 tiles fill the 256 registers of two waves per SIMD."""
+    found = {name: obj for p in ("k_gemm_prefillI", "k_gemm_prefill_subI") for name, obj in kernels(p).items()}
+    assert len(found) == 16
+    notes = subprocess.run([os.path.join(os.path.dirname(OBJDUMP), "llvm-readelf"), "--notes", next(iter(found.values()))],
+                           check=True, text=True, stdout=subprocess.PIPE).stdout
+    for name in found:
+        m = re.search(r"\.name:\s+%s\n(.*?)\.wavefront_size" % name, notes, re.S)
+        assert re.search(r"\.private_segment_fixed_size: 0\n", m.group(1)), name
+        assert re.search(r"\.vgpr_spill_count: 0\n", m.group(1)), name
