@@ -20,15 +20,16 @@
 //
 // Weights. A product's weights lie in 4 sub-blocks (the runs g), so they are scaled by their sub-blocks' integer scales
 // before it, exactly in fp16:
-//   Q4_K: sc q 2^-24 from the table's grid byte as a denormal, Q5_K: sc q (at most 63 x 31);
+//   Q4_K: sc q 2^-24 from the table's grid byte as a denormal, Q5_K: sc (q - 16) (at most 63 x 16);
 //   Q6_K, IQ4_XS: s f(q) has up to 13 bits, so s = s1 + s0 with s1 even and s0 = 1 or 2 of its sign (split_scale): s1 f(q)
-//   and s0 f(q) are exact and both products go to one accumulator. Neither part is 0 unless s is, nor do their signs
-//   differ, so an infinite activation stays infinite; IQ4_XS's kv / 16 = fp16(64 + b / 16) - 72 of the grid byte
-//   b = kv + 128, one fma per product.
+//   and s0 f(q) are exact and go into one product of k = 32 (v_mfma_f32_16x16x32_f16, as long as one of 16), each with the
+//   activations. Neither part is 0 unless s is, nor do their signs differ, so an infinite activation stays infinite;
+//   IQ4_XS's kv / 16 = fp16(64 + b / 16) - 72 of the grid byte b = kv + 128, one fma per weight pair.
 // d is applied in fp32 when the super-block is complete. Mins (Q4_K / Q5_K): one product per row group and super-block of
 // the mins with the sub-blocks' fp32 x sums, formed by launch_wide_x and held as three bf16 parts that add up to all 24
 // bits (as fp16 hi and lo a sum past 65504, 32 activations of 2047, would be infinite): parts in lane groups 0, 1 and 2 of
-// v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16.
+// v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16. Q5_K takes 16 of its codes, which lie around it, with the
+// sums as well: 16 d (sc . Sx), as exact, leaves products of sc (q - 16), whose rounding counts for less.
 // Distance from 64 bits 1.3e-7 (2-norm), against 3e-6 of the ring kernel's fp16 dot products and 2e-7 .. 8e-7 of
 // k_fused_tiles_mma.
 //
@@ -175,17 +176,29 @@ struct WideUnit {
         for (int k = 0; k < 4; ++k)
           m[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, mf[2 * k + 1]), __builtin_bit_cast(uint32_t, mf[2 * k]),
                                        0x07060302u);
-        const float off = -h2f(w[0] >> 16);
+        f4v mb = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (KQ == KQ_Q5_K) {  // the scales with the sums
+          u32x4 sb;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t v = (k < 2 ? s0 : s1) >> (16 * (k & 1));
+            sb[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, (float)(v >> 8 & 255u)),
+                                          __builtin_bit_cast(uint32_t, (float)(v & 255u)), 0x07060302u);
+          }
+          mb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, sx[a >> 1]), __builtin_bit_cast(b8v, sb), mb, 0,
+                                                       0, 0);
+        }
+        const float off = -h2f(w[0] >> 16), d16 = 16.f * h2f(w[0]);
         const f4v ma = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, sx[a >> 1]), __builtin_bit_cast(b8v, m),
                                                                f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(off, ma[r], tot[a & 1][r]);
+        for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(off, ma[r], KQ == KQ_Q5_K ? d16 * mb[r] : tot[a & 1][r]);
       }
     }
     const uint32_t rlb =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint32_t*)(buf + (lane & 15));
-    // sums of a chain (Q5_K, for the registers: of a row's two), folded into tot every 16 symbols of the 8-bit formats (one
-    // run of additions over 256 weights was 1.3 .. 1.6 times as far from 64 bits)
+    // sums of a chain (Q5_K, for the registers: of a row's two), Q6_K's folded into tot every 16 symbols (one run of
+    // additions over 256 weights was 1.3 .. 1.6 times as far from 64 bits)
     constexpr int NACC = KQ == KQ_Q5_K ? 2 : 4;
     f4v acc[NACC];
 #pragma unroll
@@ -274,25 +287,28 @@ struct WideUnit {
       }
       if constexpr (SYMB == 4 || (q & 1)) {  // 4 weights per lane
         constexpr int h = SYMB == 4 ? q & 1 : (q >> 1) & 1;
-        auto product = [&](int c, h2v sv, h2v nv) {
-          auto scaled = [&](uint32_t w) {
-            const h2v v = __builtin_bit_cast(h2v, w);
-            return __builtin_bit_cast(uint32_t, KQ == KQ_IQ4_XS ? __builtin_elementwise_fma(v, sv, nv) : v * sv);
-          };
-          const uint32_t v0 = scaled(w4[c][0]), v1 = scaled(w4[c][1]);
-          const u32x4 xp = x[st % XD][c >> 1];
-          f4v& a = acc[c % NACC];
-          a = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4v, make_uint2(xp[2 * h], xp[2 * h + 1])),
-                                                    __builtin_bit_cast(h4v, make_uint2(v0, v1)), a, 0, 0, 0);
+        auto scaled = [&](uint32_t w, h2v sv, h2v nv) {
+          h2v v = __builtin_bit_cast(h2v, w);
+          if constexpr (KQ == KQ_Q5_K) v -= dup(16.f);
+          return __builtin_bit_cast(uint32_t, KQ == KQ_IQ4_XS ? __builtin_elementwise_fma(v, sv, nv) : v * sv);
         };
 #pragma unroll
-        for (int c = 0; c < 4; ++c) product(c, s1[c], n1[c]);
-        if constexpr (SPLIT) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) product(c, s0[c], n0[c]);
+        for (int c = 0; c < 4; ++c) {
+          const u32x4 xp = x[st % XD][c >> 1];
+          const uint32_t x0 = xp[2 * h], x1 = xp[2 * h + 1];
+          const uint32_t v0 = scaled(w4[c][0], s1[c], n1[c]), v1 = scaled(w4[c][1], s1[c], n1[c]);
+          f4v& a = acc[c % NACC];
+          if constexpr (SPLIT) {  // both parts in one product, the activations twice
+            const uint32_t u0 = scaled(w4[c][0], s0[c], n0[c]), u1 = scaled(w4[c][1], s0[c], n0[c]);
+            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, make_uint4(x0, x1, x0, x1)),
+                                                       __builtin_bit_cast(h8v, make_uint4(v0, v1, u0, u1)), a, 0, 0, 0);
+          } else {
+            a = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4v, make_uint2(x0, x1)),
+                                                      __builtin_bit_cast(h4v, make_uint2(v0, v1)), a, 0, 0, 0);
+          }
         }
         if constexpr (q % PPS == PPS - 1 && st + XD < NST) load_x(st + XD);
-        if constexpr (SYMB == 8 && q != 15 && q % (KQ == KQ_Q5_K ? 4 : 8) == (KQ == KQ_Q5_K ? 3 : 7)) fold();
+        if constexpr (KQ == KQ_Q6_K && q == 7) fold();
       }
     });
     fold();

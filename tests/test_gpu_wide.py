@@ -206,3 +206,26 @@ def test_infinite_activation(gpu, lib, orc, tmp_path, kqt):
             assert err(torch.from_numpy(y[keep]), y64(orc, kqt, w["a"], x[keep])) < TOL
     finally:
         rt.close()
+
+
+@pytest.mark.parametrize("kqt", (2, 3))
+def test_short_sums_no_further_than_the_4_token_kernel(gpu, lib, orc, tmp_path, kqt):
+    """The 8-bit formats over few super-blocks, where a product's rounding shows: 16 tokens in one call are as near to fp64
+    as the same ones four by four, which the whole-tile kernel sums in integers scaled per sub-block. (Roundings of another
+    order on 16 x 1024 results: 2 % either way.)"""
+    import torch
+    rt, w = open_mats(tmp_path, [("k%d" % k, kqt, 1024, k, H[kqt], 70 + k) for k in (256, 512, 768, 1024)])
+    try:
+        for name in w:
+            K = int(name[1:])
+            x = torch.randn(16, K, generator=torch.Generator().manual_seed(K)).half().cuda()
+            y, y4 = (torch.zeros(16, 1024, device="cuda") for _ in range(2))
+            rt.matmul_dev(name, x, y)
+            for t in range(0, 16, 4):
+                rt.matmul_dev(name, x[t:t + 4], y4[t:t + 4])
+            torch.cuda.synchronize()
+            ref = y64(orc, kqt, w[name], x)
+            print("short", kqt, K, "%.3g %.3g" % (err(y, ref), err(y4, ref)), flush=True)
+            assert err(y, ref) <= 1.02 * err(y4, ref), K
+    finally:
+        rt.close()
