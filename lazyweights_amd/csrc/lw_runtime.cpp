@@ -687,22 +687,29 @@ bool wide_takes(const lw::DevMat& dm, int mt, int per) {
   return g_kernel_mode == 0 && mt <= 16 && (per == 2 ? mt >= 2 : mt >= (dm.packed ? 9 : 5)) && lw::wide_ok(dm);
 }
 
-// Its blocks (a wave per half tile; sets the entries' w and block0 and the plan's W): rows of at most 8 units whole, so
-// that a row's sum stays in the block (us per call at 5 tokens, rows of 8: q, k and v 13.3 with 8 waves, 15.0 with 4),
-// longer ones 4 units at a time, small blocks that follow each other out of step (rows of 16 and 56, Q5_K: gate + up 44.2
-// / 49.1 / 59.2 with 4 / 8 / 16, down 29.9 / 31.8 / 36.2). Every block 4 units where a CU runs many blocks one after the
-// other (a whole Q4_K layer 46.3, with 8 48.3) or the units lie in long rows mostly, or 8 buffers do not fit the LDS.
+// Its blocks (a wave per half tile; sets the entries' w and block0 and the plan's W): rows of 5 to 8 units whole, so that a
+// row's sum stays in the block, others 4 units at a time (whole rows of up to 4), small blocks that follow each other out of
+// step. us per call with blocks of 4 / of 8 waves at 5 and at 16 tokens, 28 units per CU: Q4_K rows of 8 30.7 / 29.1 and 33.5 /
+// 29.7, of 7 31.4 / 28.7 and 35.0 / 29.8, of 6 36.2 / 34.9 and 40.8 / 36.8, of 4 26.2 / 28.8 and 27.7 / 30.2, of 3 28.9 / 34.8
+// and 30.8 / 37.4, of 1 27.1 / 29.9 and 31.1 / 35.0; the same way with 4 to 80 units per CU (rows of 6 and 7: up to 5 % the
+// other way from 32 units on at 5 tokens). One block size per launch, and a block of 4 units leaves half of 8 waves idle: 8
+// where nine tenths of the units lie in such rows (three quarters, gate + up with down of 28: 40.3 / 42.2 and 45.6 / 44.4;
+// 28672 x 4096 with 1024 x 8192: 32.3 / 29.8 and 36.1 / 30.8), also for shorter rows where blocks of 8 are at most one per CU
+// and blocks of 4 more (14336 x 1536 at 16 tokens 13.4 / 12.7), and 8 buffers fit the LDS.
 void wide_blocking(lw::WidePlan& wp) {
-  long long units = 0, rows = 0;
+  long long units = 0, rows = 0, shorts = 0;
+  int n4 = 0, n8 = 0;
   for (int i = 0; i < wp.n; ++i) {
-    const long long u = 2ll * wp.e[i].M.NT * wp.e[i].M.KT;
+    const lw::DevMat& dm = wp.e[i].M;
+    const long long u = 2ll * dm.NT * dm.KT;
     units += u;
-    if (wp.e[i].M.KT <= 8) rows += u;
+    if (dm.KT <= 8) shorts += u;
+    if (dm.KT <= 8 && dm.KT > 4) rows += u;
+    n4 += lw::wide_blocks(dm, 4);
+    n8 += lw::wide_blocks(dm, 8);
   }
-  const int rows_w = 2 * rows >= units && units <= 40ll * cu_count() &&
-                             lw::wide_lds_bytes(8, lw::wide_buf_rows(wp)) <= 160 * 1024
-                         ? 8
-                         : 4;
+  const bool eight = 10 * rows >= 9 * units || (shorts == units && n4 > cu_count() && n8 <= cu_count());
+  const int rows_w = eight && lw::wide_lds_bytes(8, lw::wide_buf_rows(wp)) <= 160 * 1024 ? 8 : 4;
   int blocks = 0;
   wp.W = 1;
   for (int i = 0; i < wp.n; ++i) {
