@@ -177,7 +177,7 @@ struct WidePlan {
   WideEntry e[MAX_GROUP];
   int n, W, mt, per;
 };
-constexpr int WIDE_MAX_WAVES = 16;
+constexpr int WIDE_MAX_WAVES = 8;
 size_t wide_x_bytes(int mt, int K);  // bytes of one reordered vector
 // activations for it in one launch: job i reorders X[i] (fp16 [mt][K], any alignment; per = 2: fp32 [mt / 2][K], split
 // into hi + lo) into XT[i] (wide_x_bytes(mt, K[i]) bytes, 16-byte aligned: mt K fp16, then the sub-blocks' sums)

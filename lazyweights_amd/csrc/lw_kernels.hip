@@ -2400,7 +2400,7 @@ k_fused_halves(FlatPlan plan, int per, int ubuf_rows) {
 }
 
 // ── whole-tile kernel on the matrix cores (2..4 tokens, fp16 activations, every format) ───────────────────
-// The decode of k_fused_tiles (a tile per wave in LDS; 4 chains per lane), with the products of MT tokens on
+// The decode of k_fused_tiles (a tile per wave in LDS; 4 chains per lane), with the products of 4 token slots on
 // v_mfma_f32_4x4x4f16 (16 blocks of 4 lanes): block b computes D[i][j] = sum_k A[4 b' + i][k] B[4 b + j][k] into lane
 // 4 b + j, register i, where b' is the block named by the instruction's broadcast field (cbsz 4, abid b'). B = the
 // lane's own 4 weights of the pair (its row), A = the 4 x values of token i at those positions, broadcast from block
@@ -2415,8 +2415,8 @@ k_fused_halves(FlatPlan plan, int per, int ubuf_rows) {
 // launch to fp32 rounding (another order of the same products). Partials [KT][mt][N], the in-launch reduction.
 // The tile pipeline is k_fused_tiles': tables by direct-to-LDS loads, paced first copies, row-major tiles, the next
 // tile's copy issued as soon as a decode ends.
-// at most 16 waves per block (4 per SIMD: 128 VGPRs); 12 (3 per SIMD) for 8 tokens of the 4-bit formats, whose
-// 8 tokens' x, the 4 chains' accumulators per token quad and the chains take more than 128 VGPRs
+// At most 16 waves per block (4 per SIMD: 128 VGPRs); in the int8 form (below) 12 (3 per SIMD) for 8 tokens of the 4-bit
+// formats, whose 8 tokens' x, the 4 chains' accumulators per token quad and the chains take more than 128 VGPRs
 constexpr int TILES_MMA_WAVES = 16;
 constexpr int tiles_mma_waves(int kqt, int mt) { return mt == 8 && kq_symbits(kqt) == 4 ? 12 : TILES_MMA_WAVES; }
 
@@ -2426,15 +2426,9 @@ __device__ __forceinline__ f4v mfma4_from(h4v a, h4v b, f4v c) {
   return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, c, 4, ABID, 0);
 }
 
-template <int KQA, int NTAB, int MT, int KQB = KQA>
-__global__ void __launch_bounds__(64 * (tiles_mma_waves(KQA, MT) < tiles_mma_waves(KQB, MT) ? tiles_mma_waves(KQA, MT)
-                                                                                         : tiles_mma_waves(KQB, MT)),
-                                  1)
-k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
-  static_assert(MT == 4, "4 token slots");
-  constexpr int NQ = MT / 4;      // token quads
-  constexpr int NC = 4, NG = 16 / NC;  // chains per lane (64 symbols each: 8 tokens' x and accumulators leave no
-                                       // registers for 8 chains at 4 waves per SIMD), 16-symbol groups per chain
+template <int KQA, int NTAB, int KQB = KQA>
+__global__ void __launch_bounds__(64 * TILES_MMA_WAVES, 1) k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
+  constexpr int NC = 4, NG = 16 / NC;  // chains per lane (64 symbols each), 16-symbol groups per chain
   typedef __attribute__((address_space(3))) const uint32_t LdsU32;
   typedef __attribute__((address_space(4))) const char KChar;
   typedef __attribute__((address_space(4))) const FlatEntry KEntry;
@@ -2632,32 +2626,24 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
         for (int j = 0; j < NC; ++j) P[j] = P8[j * (8 / NC)];
       }
       const uint32_t tsel = second ? 4u * LUTN : 0u;
-      // x of the tile column: register pair m of quad q, lane 4 b + i = token 4 q + i's weights 4 (16 m + b) .. + 3
-      // (zero for tokens >= mt)
-      h4v xa[NQ][NPR], xs[NQ];
+      // x of the tile column: register pair m, lane 4 b + i = token i's weights 4 (16 m + b) .. + 3 (zero for tokens >= mt)
+      h4v xa[NPR], xs;
+      const bool ok = qi < mt;
+      const uint32_t* xrow = E.X2 + (size_t)(ok ? qi : 0) * (K / 2) + (size_t)tc * (TW / 2);
   #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        const int tok = 4 * q + qi;
-        const bool ok = tok < mt;
-        const uint32_t* xrow = E.X2 + (size_t)(ok ? tok : 0) * (K / 2) + (size_t)tc * (TW / 2);
-  #pragma unroll
-        for (int m = 0; m < NPR; ++m) {
-          const uint2 v = ok ? *reinterpret_cast<const uint2*>(xrow + 2 * (16 * m + qb)) : make_uint2(0u, 0u);
-          xa[q][m] = __builtin_bit_cast(h4v, v);
-        }
+      for (int m = 0; m < NPR; ++m) {
+        const uint2 v = ok ? *reinterpret_cast<const uint2*>(xrow + 2 * (16 * m + qb)) : make_uint2(0u, 0u);
+        xa[m] = __builtin_bit_cast(h4v, v);
       }
-      // XS: lane 4 b + i = token 4 q + i's sums of 4 sub-blocks (hi or lo halves), block b = 2 (2 sb + half) + (lo)
+      // XS: lane 4 b + i = token i's sums of 4 sub-blocks (hi or lo halves), block b = 2 (2 sb + half) + (lo)
       auto load_xs = [&]() {
-  #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          const int tok = 4 * q + qi, cb = qb & 7, lo = cb & 1, sh = cb >> 1;  // sh = 2 sb + half
-          uint64_t sv = 0;
-          if (XSUMS && tok < mt && qb < 4 * NSB) {
-            const int lc = (tc - (second ? cb0 : ca0) + KT) % KT;  // the column's slot
-            sv = xsb[(second ? xsb_b : 0) + ((size_t)lc * mt + tok) * (GPC * 2) + 2 * sh + lo];
-          }
-          xs[q] = __builtin_bit_cast(h4v, sv);
+        const int cb = qb & 7, lo = cb & 1, sh = cb >> 1;  // sh = 2 sb + half
+        uint64_t sv = 0;
+        if (XSUMS && qi < mt && qb < 4 * NSB) {
+          const int lc = (tc - (second ? cb0 : ca0) + KT) % KT;  // the column's slot
+          sv = xsb[(second ? xsb_b : 0) + ((size_t)lc * mt + qi) * (GPC * 2) + 2 * sh + lo];
         }
+        xs = __builtin_bit_cast(h4v, sv);
       };
       if (!xs_late) load_xs();
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the tile is in LDS, the pending tile's partials stored
@@ -2687,15 +2673,12 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
         const uint32_t b = (w >> (8 * (jj % 4))) & 255u;
         return (KQ == KQ_Q6_K || KQ == KQ_IQ4_XS) ? (float)(int)(int8_t)(uint8_t)b : (float)b;
       };
-      f4v acc[NC][NQ];  // per chain: its current sub-block's sums, 4 tokens per register quad
-      float fa[NQ][4];  // scaled sums of the finished sub-blocks
+      f4v acc[NC];  // per chain: its current sub-block's sums of the 4 tokens
+      float fa[4];  // scaled sums of the finished sub-blocks
   #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
+      for (int i = 0; i < 4; ++i) fa[i] = 0.f;
   #pragma unroll
-        for (int i = 0; i < 4; ++i) fa[q][i] = 0.f;
-  #pragma unroll
-        for (int j = 0; j < NC; ++j) acc[j][q] = f4v{0.f, 0.f, 0.f, 0.f};
-      }
+      for (int j = 0; j < NC; ++j) acc[j] = f4v{0.f, 0.f, 0.f, 0.f};
       uint32_t wprev[NC];
   #pragma unroll
       for (int j = 0; j < NC; ++j) wprev[j] = 0;
@@ -2730,16 +2713,12 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
                                           __builtin_amdgcn_perm(e2[j], e2[j], 0x0C030C02u));
               constexpr int g = NG * j + gi;           // 16-symbol group within the tile row
               constexpr int pb = 8 * g + p;            // position block of the 4 weights within the tile row
-  #pragma unroll
-              for (int q = 0; q < NQ; ++q)
-                acc[j][q] = mfma4_from<pb & 15>(xa[q][pb >> 4], __builtin_bit_cast(h4v, wv), acc[j][q]);
+              acc[j] = mfma4_from<pb & 15>(xa[pb >> 4], __builtin_bit_cast(h4v, wv), acc[j]);
             } else {  // 2 codes per pair (fp16(q) in the entries' upper halves), 4 per product
               const uint32_t v = __builtin_amdgcn_perm(e2[j], e1[j], 0x07060302u);
               if constexpr (p & 1) {
                 constexpr int pb = 4 * (NG * j + gi) + p / 2;
-  #pragma unroll
-                for (int q = 0; q < NQ; ++q)
-                  acc[j][q] = mfma4_from<pb & 15>(xa[q][pb >> 4], __builtin_bit_cast(h4v, make_uint2(wprev[j], v)), acc[j][q]);
+                acc[j] = mfma4_from<pb & 15>(xa[pb >> 4], __builtin_bit_cast(h4v, make_uint2(wprev[j], v)), acc[j]);
               } else {
                 wprev[j] = v;
               }
@@ -2753,19 +2732,14 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
             constexpr int js = (NG * j + gi) / GPSUB;  // sub-block within the tile row
             const float sa = dA[js / NSUB] * WSCALE * scale_of(js);
   #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-  #pragma unroll
-              for (int i = 0; i < 4; ++i) fa[q][i] = fmaf(acc[j][q][i], sa, fa[q][i]);
-              acc[j][q] = f4v{0.f, 0.f, 0.f, 0.f};
-            }
+            for (int i = 0; i < 4; ++i) fa[i] = fmaf(acc[j][i], sa, fa[i]);
+            acc[j] = f4v{0.f, 0.f, 0.f, 0.f};
           });
         }
       });
       // the products are formed here, not sunk past the claim and the copy below
   #pragma unroll
-      for (int q = 0; q < NQ; ++q)
-  #pragma unroll
-        for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(fa[q][i]));
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(fa[i]));
       if (xs_late) {  // this tile's sums, now that every share is stored
         while (__hip_atomic_load(xs_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < (uint32_t)xnw)
           __builtin_amdgcn_s_sleep(2);
@@ -2791,7 +2765,7 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
       }
       // offset terms: per super-block and token, sum_j c_j (sum x)_j from the hi and lo halves of the sums, c_j = the
       // mins m_j (Q4_K / Q5_K) or the signed scales s_j (IQ4_XS)
-      f4v mac[NSB][NQ];
+      f4v mac[NSB];
   #pragma unroll
       for (int sb = 0; sb < NSB; ++sb) {
         if constexpr (!XSUMS) break;
@@ -2804,36 +2778,30 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
         }
         const h4v m0 = h4v{(_Float16)mf[0], (_Float16)mf[1], (_Float16)mf[2], (_Float16)mf[3]};
         const h4v m1 = h4v{(_Float16)mf[4], (_Float16)mf[5], (_Float16)mf[6], (_Float16)mf[7]};
-  #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-          f4v r = {0.f, 0.f, 0.f, 0.f};
-          if (sb == 0) {
-            r = mfma4_from<0>(xs[q], m0, r);
-            r = mfma4_from<1>(xs[q], m0, r);
-            r = mfma4_from<2>(xs[q], m1, r);
-            r = mfma4_from<3>(xs[q], m1, r);
-          } else {
-            r = mfma4_from<4>(xs[q], m0, r);
-            r = mfma4_from<5>(xs[q], m0, r);
-            r = mfma4_from<6>(xs[q], m1, r);
-            r = mfma4_from<7>(xs[q], m1, r);
-          }
-          mac[sb][q] = r;
+        f4v r = {0.f, 0.f, 0.f, 0.f};
+        if (sb == 0) {
+          r = mfma4_from<0>(xs, m0, r);
+          r = mfma4_from<1>(xs, m0, r);
+          r = mfma4_from<2>(xs, m1, r);
+          r = mfma4_from<3>(xs, m1, r);
+        } else {
+          r = mfma4_from<4>(xs, m0, r);
+          r = mfma4_from<5>(xs, m0, r);
+          r = mfma4_from<6>(xs, m1, r);
+          r = mfma4_from<7>(xs, m1, r);
         }
+        mac[sb] = r;
       }
       float* out = E.P + (size_t)tc * mt * N + (size_t)tr * TN + (uint32_t)lane;
   #pragma unroll
-      for (int q = 0; q < NQ; ++q)
+      for (int i = 0; i < 4; ++i) {
+        float tot = fa[i];
+        if constexpr (XSUMS) {
   #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float tot = fa[q][i];
-          if constexpr (XSUMS) {
-  #pragma unroll
-            for (int sb = 0; sb < NSB; ++sb)
-              tot = fmaf(KQ == KQ_IQ4_XS ? -128.f * dA[sb] : -dB[sb], mac[sb][q][i], tot);
-          }
-          if (4 * q + i < mt) __hip_atomic_store(out + (size_t)(4 * q + i) * N, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int sb = 0; sb < NSB; ++sb) tot = fmaf(KQ == KQ_IQ4_XS ? -128.f * dA[sb] : -dB[sb], mac[sb][i], tot);
         }
+        if (i < mt) __hip_atomic_store(out + (size_t)i * N, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       if (pend >= 0 && old == (uint32_t)(pKT - 1)) row_sum(*(pend ? eb : ea), ptr, pKT, pN, lane, mt);
       pend = -1;
       if (E.Y) {
@@ -2857,14 +2825,14 @@ k_fused_tiles_mma(FlatPlan plan, int per, int buf_rows) {
   }
 }
 
-template <int KQ, int NTAB, int MT, int KQB = KQ>
+template <int KQ, int NTAB, int KQB = KQ>
 static hipError_t tiles_mma_launch_t(const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
   const size_t smem = (size_t)p.W * buf_rows * 128 + tiles_mma_xs_bytes(p, per);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused_tiles_mma<KQ, NTAB, MT, KQB>),
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused_tiles_mma<KQ, NTAB, KQB>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return e;
   const int blocks = (p.ntiles + per - 1) / per;
-  hipLaunchKernelGGL((k_fused_tiles_mma<KQ, NTAB, MT, KQB>), dim3(blocks), dim3(p.W * 64), smem, s, p, per,
+  hipLaunchKernelGGL((k_fused_tiles_mma<KQ, NTAB, KQB>), dim3(blocks), dim3(p.W * 64), smem, s, p, per,
                      buf_rows);
   return hipGetLastError();
 }
@@ -2872,7 +2840,7 @@ static hipError_t tiles_mma_launch_t(const FlatPlan& p, int per, int buf_rows, h
 // two K-quant types in one launch: entries [0, nfa) of type KQA < KQB, the rest of KQB
 template <int KQA, int KQB>
 static hipError_t tiles_mma_launch_mixed_t(const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
-  return tiles_mma_launch_t<KQA, 2, 4, KQB>(p, per, buf_rows, s);
+  return tiles_mma_launch_t<KQA, 2, KQB>(p, per, buf_rows, s);
 }
 static hipError_t tiles_mma_launch_mixed(int kqa, int kqb, const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
   switch (kqa * 8 + kqb) {
@@ -2888,7 +2856,7 @@ static hipError_t tiles_mma_launch_mixed(int kqa, int kqb, const FlatPlan& p, in
 
 template <int KQ>
 static hipError_t tiles_mma_launch(const FlatPlan& p, int per, int buf_rows, hipStream_t s) {
-  return p.n == 1 ? tiles_mma_launch_t<KQ, 1, 4>(p, per, buf_rows, s) : tiles_mma_launch_t<KQ, 2, 4>(p, per, buf_rows, s);
+  return p.n == 1 ? tiles_mma_launch_t<KQ, 1>(p, per, buf_rows, s) : tiles_mma_launch_t<KQ, 2>(p, per, buf_rows, s);
 }
 
 // ── whole-tile kernel on the matrix cores for int8 activations (2..8 tokens, every format) ─────────────────
