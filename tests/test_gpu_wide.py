@@ -9,7 +9,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# fp32 sums of exact products, K <= 28672 terms in sums of 16: 2-norm errors of a few 2^-24
+# fp32 sums of exact products, K <= 14336 terms in sums of 16: 2-norm errors of a few 2^-24
 TOL = 1e-6
 H = {1: 2.3, 2: 3.4, 3: 4.3, 4: 2.6}
 
@@ -229,3 +229,40 @@ def test_short_sums_no_further_than_the_4_token_kernel(gpu, lib, orc, tmp_path, 
             assert err(y, ref) <= 1.02 * err(y4, ref), K
     finally:
         rt.close()
+
+
+@pytest.mark.parametrize("kqt", (1, 2, 3, 4))
+def test_block_sizes_and_uneven_tiles(gpu, lib, orc, tmp_path, kqt):
+    """Rows of 6 units (whole, blocks of 6 waves), of 2 and 3 where blocks of 8 waves are at most one per CU and blocks of 4
+    more (a last block with rows left over), and tiles whose halves and rows differ in length: runs of the most frequent
+    code beside uniform codes."""
+    import torch
+    from lazyweights_amd import Runtime
+    from lazyweights_amd.bundle import Writer, synth_matrix
+    cols, ncodes = (512, 16) if kqt in (1, 4) else (256, 32 if kqt == 2 else 64)
+    rng = np.random.default_rng(kqt)
+    w, out = Writer(str(tmp_path)), {}
+    for name, N, units in (("six", 192, 6), ("two", 64 * 301, 2), ("three", 64 * 151, 3), ("uneven", 256, 9)):
+        codes, side = synth_matrix(kqt, N, units * cols, H[kqt], 80 + units, threads=16)
+        if name == "uneven":
+            codes[:] = ncodes // 2
+            for r0 in (0, 40, 96, 128, 200):  # 8 to 32 long rows in the one half or the other, the rest a bit per symbol
+                codes[r0:r0 + 8 + r0 % 25] = rng.integers(0, ncodes, (8 + r0 % 25, units * cols))
+        w.add_kquant(name, kqt, codes, side)
+        out[name] = (codes, side)
+    w.close()
+    with Runtime(tmp_path) as rt:
+        for name, (codes, side) in out.items():
+            N, K = codes.shape
+            d = orc.dequant(kqt, codes, side).astype(np.float64)
+            for m, f16 in ((5, True), (16, True), (3, False)):
+                x = torch.randn(m, K, generator=torch.Generator().manual_seed(m))
+                x = (x.half() if f16 else x).cuda()
+                y = torch.full((m, N), float("nan"), device="cuda")
+                for _ in range(2):
+                    rt.matmul_dev(name, x, y, x_f16=f16)
+                torch.cuda.synchronize()
+                ref = x.double().cpu().numpy() @ d.T
+                e = err(y, ref)
+                print("blocks", name, kqt, N, K, m, f16, "err %.2g" % e, flush=True)
+                assert e < TOL, (name, m)
