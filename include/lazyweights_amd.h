@@ -36,7 +36,9 @@ void rt_close(void* h);
 int rt_test_matmul(void* h, const char* name, const float* X, int m, float* Y, int path);
 
 /* Replaces rt_test_decode (kernels/llmrt.cu:2461): GPU decode to host codes [N, K] (one byte per weight, pair
- * symbols unpacked low nibble first, no add for K-quants); raw8 tensors are copied. -1 if not resident. */
+ * symbols unpacked low nibble first, no add for K-quants); raw8 tensors are copied. -1 if not resident. The first call
+ * keeps up to 64 MB of device memory (the largest matrix's codes, at most) and 16 MB of pinned host memory with the
+ * handle until rt_close; calls that overlap on one handle take them in turn. */
 int rt_test_decode(void* h, const char* name, uint8_t* out);
 
 /* Replaces rt_gpu_decode_all (kernels/llmrt.cu:2482): GPU decode of every resident coded matrix; median seconds of
@@ -79,8 +81,9 @@ int lw_tensor_info(void* h, const char* name, int64_t* out);
 /* Device-pointer GEMV / skinny GEMM on `stream` (a hipStream_t; NULL = the null stream), no host copies, no
  * synchronisation: Y[m, N] (row stride ldy) = X[m, K] @ dequant(W)^T. X is fp16 (x_f16 = 1, the headline path,
  * m <= 16) or fp32 (x_f16 = 0: split into fp16 hi + lo; m <= 8 fused, any larger m the prefill path: decode into a
- * device scratch and GEMMs on the matrix cores, as rt_test_matmul's path 2, see lw_set_prefill_gemm). Returns 0 or
- * -1. */
+ * device scratch and GEMMs on the matrix cores, as rt_test_matmul's path 2, see lw_set_prefill_gemm). fp32 activations
+ * must lie within fp16's range (65504), and with Q4_K and Q5_K at m > 8 (fp16: Q4_K, Q5_K and IQ4_XS at 2 <= m <= 4)
+ * also the sums of 32 that share a sub-block; results past it are not finite. Returns 0 or -1. */
 int lw_matmul_dev(void* h, const char* name, const void* X, int x_f16, int m, float* Y, int ldy, void* stream);
 
 /* lw_matmul_dev without any device allocation. No counterpart in the reference: it is for callers that cannot
@@ -89,7 +92,9 @@ int lw_matmul_dev(void* h, const char* name, const void* X, int x_f16, int m, fl
  * runs on until the process ends; the counters are cleared by a kernel on `stream` at each call. Fused path only:
  * fp16 X with 1 <= m <= 16 or fp32 X with 1 <= m <= 8, int8 activations off; -1 with an error text when the call
  * needs more than the 16 MiB (KT * m * N * 4 bytes of partials, 8 with fp32 X, + 8 * N / 64 of counters + 4 m K of
- * split x). Calls that overlap on one GPU (several streams or threads) race on the array. */
+ * split x). The 16-token kernel's reordered activations take what these leave, or the partials it does not need; a call
+ * where neither has room for them (a few hundred rows of some 100000 weights, or a quarter of a million rows of one tile)
+ * goes through the ring kernels and gives their bits. Calls that overlap on one GPU (several streams or threads) race on the array. */
 int lw_matmul_dev_noalloc(void* h, const char* name, const void* X, int x_f16, int m, float* Y, int ldy,
                           void* stream);
 
@@ -119,11 +124,11 @@ int lw_group_matmul_dev(void* h, int count, const char* const* names, const void
 int lw_set_kernel_mode(int mode);
 
 /* Prefill GEMM (path 2, and fp32 X with m > 8) for every handle. The reference dequantizes to fp32 and runs its own
- * fp32 GEMM (kernels/llmrt.cu:201-343, 1826-1841). 0 (default) = the hand-written matrix-core GEMM for Q4_K / Q5_K
- * (codes decoded to a device scratch, each scaled by its 6-bit sub-block scale into an exact fp16 weight, x split into
- * fp16 hi + lo, v_mfma_f32_32x32x16_f16 with fp32 accumulation, super-block scales and mins applied in registers) and
- * rocBLAS for Q6_K / IQ4_XS; 1 = hand-written for every format (Q6_K / IQ4_XS through a per-sub-block-scaled MFMA
- * GEMM); 2 / 3 = rocBLAS always, over the decoded weights w = s f(q) - o split into fp16 hi + lo (two fp16 GEMMs with
+ * fp32 GEMM (kernels/llmrt.cu:201-343, 1826-1841). 0 (default) = the hand-written matrix-core GEMMs over codes decoded to
+ * a device scratch in a tiled layout, x split into fp16 hi + lo, v_mfma_f32_32x32x16_f16 with fp32 accumulation: Q4_K /
+ * Q5_K with each code scaled by its 6-bit sub-block scale into an exact fp16 weight, super-block scales and mins applied
+ * in registers, Q6_K / IQ4_XS with the grid values, each sub-block's sums scaled in fp32; 1 = the older hand-written GEMM
+ * over row-major codes for every format; 2 / 3 = rocBLAS always, over the decoded weights w = s f(q) - o split into fp16 hi + lo (two fp16 GEMMs with
  * fp32 accumulation, x_hi w_hi + x_hi w_lo, then + x_lo w_hi / one GEMM over 2m columns [x_hi | x_hi] and [x_lo | 0]);
  * 4 = rocBLAS with the one-GEMM form up to 512 tokens. Kernel mode 1 overrides all with the SIMT GEMM. Returns 0 or
  * -1. */

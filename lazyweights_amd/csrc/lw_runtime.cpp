@@ -680,7 +680,9 @@ int halves_width(const lw::FlatPlan& fp, int mintiles, int& per) {
 // that a matrix gives the same bits in a group and on its own. For 2..4 fp16 tokens k_fused_tiles_mma stays: us per call
 // against this kernel, Q4_K gate + up 29.3 / 29.5 at 2 tokens, 31.0 / 29.4 at 4, 31.6 / 29.2 at 5, 36.2 / 29.4 at 8, a
 // whole layer 43.5 / 46, 47.5 / 46, 52.5 / 46.3, 59.6 / 47; Q5_K gate + up 38.2 / 44.2 at 2, 44.0 / 44.2 at 5 (its waves
-// take tile after tile, so many tiles per CU cost it one start; with few per CU this kernel is ahead at 2 as well).
+// take tile after tile, so many tiles per CU cost it one start; with few per CU this kernel is ahead at 2 as well). fp32 x of
+// one and two tokens, which only the ring kernels took before: Q4_K 4096 x 14336 34.8 / 19.5 and 32.9 / 19.6, 1024 x 4096
+// 30.4 / 12.3 and 29.1 / 12.3, Q6_K 4096 x 14336 35.7 / 29.0 and 33.7 / 29.0.
 // A packed matrix takes it with fp32 x and from 9 fp16 tokens, which keeps a twin at the coded matrix's bits there; up to 8
 // fp16 tokens it has those of the ring kernels (kernel mode 7).
 bool wide_takes(const lw::DevMat& dm, int mt, int per) {
@@ -1525,7 +1527,8 @@ uint8_t* scratch_on_device() {
   return static_cast<uint8_t*>(p);
 }
 
-// Device bytes to a caller's ordinary host memory, after the work on M.stream: pieces through pinned memory, copied out
+// Device bytes to a caller's ordinary host memory, after the work on M.stream: pieces through pinned memory (kept by the
+// handle, 16 MB), copied out
 // by kCopyThreads threads while later pieces arrive. A plain copy into memory the caller has just allocated runs at the
 // rate one thread takes page faults (16.8 MB: 1250 us, of which 310 us are the transfer; a pinned transfer and 4 threads
 // touching the pages: 340-430 us side by side; this: 756 us a call, 515 into memory touched before. 8 threads, or pieces of

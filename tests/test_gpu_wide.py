@@ -124,7 +124,7 @@ def test_sub_block_sums_past_fp16(gpu, lib, orc, tmp_path, kqt):
     rt, w = open_mats(tmp_path, [("a", kqt, 192, 4608, H[kqt], 31)])
     try:
         d = orc.dequant(kqt, *w["a"])
-        for m, f16 in ((5, True), (9, True), (16, True), (1, False), (8, False)):
+        for m, f16 in ((1, True), (5, True), (9, True), (16, True), (1, False), (8, False)):
             x = torch.randn(m, 4608, generator=torch.Generator().manual_seed(m))
             x[0, 96:128] = 3000
             x[m // 2, [512, 540]] = 40000
