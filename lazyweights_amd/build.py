@@ -174,11 +174,11 @@ def build(verbose=False):
 
 
 def build_timeline(verbose=False):
-    """The diagnostic library (lazyweights_amd.timeline): the same sources, the device code compiled with
+    """The diagnostic library (lazyweights_amd.timeline): the same sources, lw_kernels.hip compiled with
     -DLW_TIMELINE (per-wave timestamps in the whole-tile kernel), beside the product library. Builds the product's
-    host objects first if they are missing."""
+    other objects first if they are missing."""
     os.makedirs(BUILD, exist_ok=True)
-    objs = [os.path.join(BUILD, os.path.splitext(src)[0] + ".o") for src, kind in SOURCES if kind != "hip"]
+    objs = [os.path.join(BUILD, os.path.splitext(src)[0] + ".o") for src, _ in SOURCES if src != "lw_kernels.hip"]
     if not all(os.path.exists(o) for o in objs):
         build()
     obj = os.path.join(BUILD, "lw_kernels_timeline.o")

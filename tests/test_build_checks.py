@@ -145,3 +145,16 @@ def test_prefill_gemm_keeps_its_tiles_in_registers(kernels):
         m = re.search(r"\.name:\s+%s\n(.*?)\.wavefront_size" % name, notes, re.S)
         assert re.search(r"\.private_segment_fixed_size: 0\n", m.group(1)), name
         assert re.search(r"\.vgpr_spill_count: 0\n", m.group(1)), name
+
+
+def test_timeline_build_links_every_object(monkeypatch):
+    """The diagnostic library holds the objects of every source, lw_kernels.hip's compiled anew."""
+    from lazyweights_amd import build
+    ran = []
+    monkeypatch.setattr(build, "_run", lambda cmd: ran.append(cmd))
+    monkeypatch.setattr(build, "check_dpp_hazards", lambda lib: 1)
+    monkeypatch.setattr(build.os, "replace", lambda a, b: None)
+    monkeypatch.setattr(build.os.path, "exists", lambda p: True)
+    build.build_timeline()
+    objs = {os.path.basename(a) for a in ran[-1] if a.endswith(".o")}
+    assert objs == {os.path.splitext(src)[0] + ".o" for src, _ in build.SOURCES} - {"lw_kernels.o"} | {"lw_kernels_timeline.o"}
