@@ -48,6 +48,7 @@ struct DevMat {
   int nexc, nexc32;
   // 1: a packed (fixed-rate) matrix: words = the symbols as 16-byte chunks [T][16][64], lut4 = 256 symbol entries
   int packed;
+  int centre;  // Q5_K: the mean code, rounded (what the 16-token kernel takes off every code); else 0
 };
 
 // Matrices of one grouped launch of the ring kernel (same K-quant type and ring size). Matrix i owns blocks

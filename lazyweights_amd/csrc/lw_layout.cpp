@@ -36,15 +36,16 @@ static void parallel_for(int n, int threads, const std::function<void(int, int)>
 namespace {
 
 // Decode one lane (512 symbols) from a bit source: bits32(off) = 32 stream bits from lane offset `off`.
-// pos[i] = lane bit offset before symbol i (i = 0..512). Fails if the lane runs past `limit` bits.
+// pos[i] = lane bit offset before symbol i (i = 0..512); sum += the symbols. Fails if the lane runs past `limit` bits.
 template <class B>
-inline bool decode_lane(const uint16_t* lut, B bits32, uint64_t limit, uint32_t* pos) {
+inline bool decode_lane(const uint16_t* lut, B bits32, uint64_t limit, uint32_t* pos, uint64_t& sum) {
   uint64_t bp = 0;
   for (int i = 0; i < LANE_SYMS; ++i) {
     pos[i] = (uint32_t)bp;
     if (bp >= limit) return false;
     const uint16_t e = lut[bits32(bp) & (LUTN - 1)];
     bp += e >> 8;
+    sum += e & 255u;
   }
   pos[LANE_SYMS] = (uint32_t)bp;
   return bp <= limit;
@@ -124,12 +125,14 @@ bool analyse_tiles(Layout& L, int T, int threads, B bits32, Lim limit, Check che
   lane_bits.assign((size_t)T * LANES, 0);
   std::vector<uint8_t> ring_ok(T, 0);  // bit 0: RS 16 fits, bit 1: RS 32 fits
   std::atomic<bool> bad(false);
+  std::atomic<uint64_t> symbol_sum(0);
   parallel_for(T, threads, [&](int t0, int t1) {
     std::vector<uint32_t> pos((size_t)LANES * (LANE_SYMS + 1));
+    uint64_t sum = 0;
     for (int t = t0; t < t1 && !bad; ++t) {
       for (int l = 0; l < LANES; ++l) {
         uint32_t* p = pos.data() + (size_t)l * (LANE_SYMS + 1);
-        if (!decode_lane(L.lut, [&](uint64_t off) { return bits32(t, l, off); }, limit(t, l), p) ||
+        if (!decode_lane(L.lut, [&](uint64_t off) { return bits32(t, l, off); }, limit(t, l), p, sum) ||
             !check_end(t, l, p[LANE_SYMS])) {
           bad = true;
           break;
@@ -206,7 +209,9 @@ bool analyse_tiles(Layout& L, int T, int threads, B bits32, Lim limit, Check che
         L.sched[2 * (size_t)t + 1] = (uint64_t)base_used | (uint64_t)init[0] << 8 | (uint64_t)init[1] << 16;
       }
     }
+    symbol_sum += sum;
   });
+  L.symbol_sum = symbol_sum;
   if (bad) return false;
   // one ring size per matrix: 16 rows when at most 1/32 of the tiles need the whole-tile fallback, else 32 if
   // every tile fits, else none (whole-tile kernel for the matrix)

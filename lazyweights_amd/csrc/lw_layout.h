@@ -51,6 +51,7 @@ struct Layout {
   int tstride = 0;
   int max_hrows = 0;  // max over tiles and halves of a half-tile unit's rows
   uint64_t payload_bits = 0;    // coded bits of all lanes
+  uint64_t symbol_sum = 0;      // of all symbols
 };
 
 // From a raw huf8/huf4p blob (lazyweights/bundle.py:14-21). N rows, KS symbols per row. Every lane is decoded once

@@ -269,6 +269,12 @@ bool upload_side(Model& M, Tensor& t) {
   return true;
 }
 
+// DevMat::centre from the sum of a matrix's symbols
+int mean_code(const Tensor& t, uint64_t symbol_sum) {
+  const uint64_t n = (uint64_t)t.N * t.KS();
+  return t.kqt == lw::KQ_Q5_K ? (int)std::min<uint64_t>((symbol_sum + n / 2) / n, 31) : 0;
+}
+
 // Build and upload the device layout (and side bytes) of a coded tensor.
 bool make_resident(Model& M, Tensor& t, int threads) {
   std::vector<uint8_t> blob(t.nbytes + 16, 0);
@@ -377,6 +383,7 @@ bool make_resident(Model& M, Tensor& t, int threads) {
   dm.max_rows = L.max_rows;
   dm.tstride = L.tstride;
   dm.max_hrows = L.max_hrows;
+  dm.centre = mean_code(t, L.symbol_sum);
   if (t.kqt && !upload_side(M, t)) return false;
   t.resident = true;
   M.resident_bytes += bytes + t.side_bytes;
@@ -405,6 +412,8 @@ bool make_resident_packed(Model& M, Tensor& t) {
     lw::decode_table_i8(t.kqt, ident.data(), tab.data());
     memcpy(host.data() + 256 * 4, tab.data(), 256 * 4);
   }
+  uint64_t symbol_sum = 0;
+  for (const uint8_t v : blob) symbol_sum += v;
   uint8_t* w = host.data() + o_words;
   for (int tr = 0; tr < NT; ++tr)
     for (int tc = 0; tc < KT; ++tc)
@@ -438,6 +447,7 @@ bool make_resident_packed(Model& M, Tensor& t) {
   dm.symbits = t.symbits;
   dm.KT = KT;
   dm.NT = NT;
+  dm.centre = mean_code(t, symbol_sum);
   if (t.kqt && !upload_side(M, t)) return false;
   t.resident = true;
   M.resident_bytes += bytes + t.side_bytes;

@@ -20,7 +20,7 @@
 //
 // Weights. A product's weights lie in 4 sub-blocks (the runs g), so they are scaled by their sub-blocks' integer scales
 // before it, exactly in fp16:
-//   Q4_K: sc q 2^-24 from the table's grid byte as a denormal, Q5_K: sc (q - 16) (at most 63 x 16);
+//   Q4_K: sc q 2^-24 from the table's grid byte as a denormal, Q5_K: sc (q - c) (at most 63 x 31);
 //   Q6_K, IQ4_XS: s f(q) has up to 13 bits, so s = s1 + s0 with s1 even and s0 = 1 or 2 of its sign (split_scale): s1 f(q)
 //   and s0 f(q) are exact and go into one product of k = 32 (v_mfma_f32_16x16x32_f16, as long as one of 16), each with the
 //   activations. Neither part is 0 unless s is, nor do their signs differ, so an infinite activation stays infinite;
@@ -28,8 +28,9 @@
 // d is applied in fp32 when the super-block is complete. Mins (Q4_K / Q5_K): one product per row group and super-block of
 // the mins with the sub-blocks' fp32 x sums, formed by launch_wide_x and held as three bf16 parts that add up to all 24
 // bits (as fp16 hi and lo a sum past 65504, 32 activations of 2047, would be infinite): parts in lane groups 0, 1 and 2 of
-// v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16. Q5_K takes 16 of its codes, which lie around it, with the
-// sums as well: 16 d (sc . Sx), as exact, leaves products of sc (q - 16), whose rounding counts for less.
+// v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16. Q5_K takes its mean code c
+// (DevMat::centre) off every code and with the sums instead: c d (sc . Sx), as exact, leaves products of sc (q - c), whose
+// rounding counts for less.
 // Distance from 64 bits 1.3e-7 (2-norm), against 3e-6 of the ring kernel's fp16 dot products and 2e-7 .. 8e-7 of
 // k_fused_tiles_mma.
 //
@@ -143,7 +144,7 @@ struct WideUnit {
 
   // results [16 tokens][32 rows] of the unit in tot[i][r] (token 4 g + r, row 16 i + j); buf: its word rows in LDS, row
   // 0 of the buffer the tile's row r0
-  __device__ __forceinline__ void decode(const uint32_t* buf, int r0, int lane, f4v (&tot)[2]) {
+  __device__ __forceinline__ void decode(const uint32_t* buf, int r0, int lane, int centre, f4v (&tot)[2]) {
     const int g = lane >> 4;
     // the sub-block scales of the runs of chains 2 p and 2 p + 1 (two bytes each; Q5_K one of them) and d of rows
     // 0 and 1 of a super-block, two to a word
@@ -188,11 +189,11 @@ struct WideUnit {
           mb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, sx[a >> 1]), __builtin_bit_cast(b8v, sb), mb, 0,
                                                        0, 0);
         }
-        const float off = -h2f(w[0] >> 16), d16 = 16.f * h2f(w[0]);
+        const float off = -h2f(w[0] >> 16), dc = (float)centre * h2f(w[0]);
         const f4v ma = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8v, sx[a >> 1]), __builtin_bit_cast(b8v, m),
                                                                f4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(off, ma[r], KQ == KQ_Q5_K ? d16 * mb[r] : tot[a & 1][r]);
+        for (int r = 0; r < 4; ++r) tot[a & 1][r] = fmaf(off, ma[r], KQ == KQ_Q5_K ? dc * mb[r] : tot[a & 1][r]);
       }
     }
     const uint32_t rlb =
@@ -289,7 +290,7 @@ struct WideUnit {
         constexpr int h = SYMB == 4 ? q & 1 : (q >> 1) & 1;
         auto scaled = [&](uint32_t w, h2v sv, h2v nv) {
           h2v v = __builtin_bit_cast(h2v, w);
-          if constexpr (KQ == KQ_Q5_K) v -= dup(16.f);
+          if constexpr (KQ == KQ_Q5_K) v -= dup((float)centre);
           return __builtin_bit_cast(uint32_t, KQ == KQ_IQ4_XS ? __builtin_elementwise_fma(v, sv, nv) : v * sv);
         };
 #pragma unroll
@@ -384,7 +385,7 @@ k_fused_wide(WidePlan plan, int buf_rows) {
                                          0, 0);
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (have) unit.decode(buf, r0, lane, tot);
+    if (have) unit.decode(buf, r0, lane, e->M.centre, tot);
   };
   const int kqt = KQ ? KQ : e->M.kqt;
   if (kqt == KQ_Q4_K) run(WideTag<KQ_Q4_K>{});

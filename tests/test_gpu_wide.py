@@ -266,3 +266,39 @@ def test_block_sizes_and_uneven_tiles(gpu, lib, orc, tmp_path, kqt):
                 e = err(y, ref)
                 print("blocks", name, kqt, N, K, m, f16, "err %.2g" % e, flush=True)
                 assert e < TOL, (name, m)
+
+
+@pytest.mark.parametrize("ends", ("low", "high", "zeros"))
+def test_one_sided_codes(gpu, lib, orc, tmp_path, ends):
+    """Q5_K codes that lie at an end of their range: what the kernel takes off every code follows them (16 for all of them
+    put such results up to 25 times as far from fp64 as the 4-token kernel's), and a packed twin, whose codes are the same,
+    has the bits. Bound, in squares of a rounding at the result's size: a unit's one run of 16 additions rounds 1/16 + .. +
+    16/16 = 8.5, where the rest of the codes makes up the whole result, its fold and sums 3; the 4-token kernel's 8 folds
+    per super-block 4.5 and its sum 1: the square root of 11.5 / 5.5 is 1.45."""
+    import torch
+    from lazyweights_amd import Runtime
+    from lazyweights_amd.bundle import Writer, synth_matrix
+    rng = np.random.default_rng(9)
+    out = {}
+    for d in ("coded", "packed"):
+        w = Writer(str(tmp_path / d))
+        for K in (1024, 4096):
+            if d == "coded":
+                _, side = synth_matrix(2, 512, K, H[2], 90, threads=16)
+                codes = np.minimum(rng.geometric(0.8 if ends == "zeros" else 0.35, (512, K)) - 1, 31).astype(np.uint8)
+                out[K] = (31 - codes if ends == "high" else codes, side)
+            w.add_kquant("k%d" % K, 2, *out[K], packed=d == "packed")
+        w.close()
+    with Runtime(tmp_path / "coded") as rc, Runtime(tmp_path / "packed") as rp:
+        for K in out:
+            x = torch.randn(16, K, generator=torch.Generator().manual_seed(K)).half().cuda()
+            y, y4, yp = (torch.zeros(16, 512, device="cuda") for _ in range(3))
+            rc.matmul_dev("k%d" % K, x, y)
+            rp.matmul_dev("k%d" % K, x, yp)
+            for t in range(0, 16, 4):
+                rc.matmul_dev("k%d" % K, x[t:t + 4], y4[t:t + 4])
+            torch.cuda.synchronize()
+            ref = y64(orc, 2, out[K], x)
+            print("one-sided", ends, K, "%.3g %.3g" % (err(y, ref), err(y4, ref)), flush=True)
+            assert err(y, ref) <= 1.45 * err(y4, ref), K
+            assert torch.equal(y, yp)
