@@ -18,6 +18,7 @@ namespace lw {
 struct DevMat {
   const uint16_t* lut;
   const uint32_t* lut4;  // the ring kernels' 4-byte table entries (decode_table4 in lw_layout.h); null if kqt == 0
+  const uint32_t* lutw;  // the 16-token kernel's: lut4, for Q5_K a table of its own (centre)
   const uint32_t* luti8; // the same with int8 grid values (decode_table_i8), for int8 activations
   const uint32_t* canon; // the comparator form of lut4 (canon_table in lw_layout.h); null if the codes are not canonical
   const uint32_t* tbase;
@@ -48,7 +49,7 @@ struct DevMat {
   int nexc, nexc32;
   // 1: a packed (fixed-rate) matrix: words = the symbols as 16-byte chunks [T][16][64], lut4 = 256 symbol entries
   int packed;
-  int centre;  // Q5_K: the mean code, rounded (what the 16-token kernel takes off every code); else 0
+  int centre;  // Q5_K: the mean code, rounded, which lutw takes off every code; else 0
 };
 
 // Matrices of one grouped launch of the ring kernel (same K-quant type and ring size). Matrix i owns blocks

@@ -492,7 +492,7 @@ bool cpu_decode(const uint8_t* blob, size_t nbytes, int N, int KS, int threads, 
 
 namespace lw {
 
-void decode_table4(int kqt, const uint16_t* lut, uint32_t* out) {
+void decode_table4(int kqt, const uint16_t* lut, uint32_t* out, int centre) {
   for (int i = 0; i < LUTN; ++i) {
     const uint32_t sym = lut[i] & 255u, len = lut[i] >> 8;
     uint32_t v = len;
@@ -501,7 +501,7 @@ void decode_table4(int kqt, const uint16_t* lut, uint32_t* out) {
       if (kqt == KQ_IQ4_XS) v |= (uint32_t)(IQ4_GRID[lo] + 128) << 16 | (uint32_t)(IQ4_GRID[hi] + 128) << 24;
       else v |= lo << 16 | hi << 24;
     } else {
-      const float g = kqt == KQ_Q6_K ? (float)sym - 32.f : (float)sym;
+      const float g = kqt == KQ_Q6_K ? (float)sym - 32.f : (float)sym - (float)centre;
       v |= (uint32_t)f32_to_f16(g) << 16;
     }
     out[i] = v;

@@ -286,11 +286,11 @@ bool make_resident(Model& M, Tensor& t, int threads) {
   if (!ok) return fail(t.name + ": " + err);
   std::vector<uint8_t>().swap(blob);
   const int T = t.T();
-  // [lut 4096 B][4-byte table 8192 B][int8 table 8192 B][comparator table 1152 B][tbase 4T][mid 64T][split 1024T][rows 2T]
+  // [lut 4096 B][4-byte table 8192 B][int8 table 8192 B][comparator table 1152 B][Q5_K: lutw 8192 B][tbase 4T][mid 64T][split 1024T][rows 2T]
   // [sched 16T (16-aligned)][hrow 4T][hsplit 1024T][dsplit 512T][exception tiles 4E] padded to 256 B, then the words
   const size_t nexc = L.exc.size();
   const size_t o_lut4 = 2 * lw::LUTN, o_luti8 = o_lut4 + 4 * lw::LUTN, o_canon = o_luti8 + 4 * lw::LUTN;
-  const size_t o_tb = o_canon + 4 * lw::CANON_WORDS;
+  const size_t o_lutw = o_canon + 4 * lw::CANON_WORDS, o_tb = o_lutw + (t.kqt == lw::KQ_Q5_K ? 4 * lw::LUTN : 0);
   const size_t o_mid = o_tb + 4ull * T;
   const size_t o_split = o_mid + 64ull * T, o_rows = o_split + 64ull * lw::SPLITS * T;
   const size_t o_sched = (o_rows + 2ull * T + 15) & ~(size_t)15, o_hrow = o_sched + 16ull * T;
@@ -304,6 +304,8 @@ bool make_resident(Model& M, Tensor& t, int threads) {
   if (t.kqt) {
     lw::decode_table4(t.kqt, L.lut, reinterpret_cast<uint32_t*>(host.data() + o_lut4));
     lw::decode_table_i8(t.kqt, L.lut, reinterpret_cast<uint32_t*>(host.data() + o_luti8));
+    if (t.kqt == lw::KQ_Q5_K)
+      lw::decode_table4(t.kqt, L.lut, reinterpret_cast<uint32_t*>(host.data() + o_lutw), mean_code(t, L.symbol_sum));
     canon = lw::canon_table(L.lut, reinterpret_cast<const uint32_t*>(host.data() + o_lut4),
                             reinterpret_cast<uint32_t*>(host.data() + o_canon));
   }
@@ -357,6 +359,7 @@ bool make_resident(Model& M, Tensor& t, int threads) {
   uint8_t* b = static_cast<uint8_t*>(d);
   dm.lut = reinterpret_cast<const uint16_t*>(b);
   dm.lut4 = t.kqt ? reinterpret_cast<const uint32_t*>(b + o_lut4) : nullptr;
+  dm.lutw = t.kqt == lw::KQ_Q5_K ? reinterpret_cast<const uint32_t*>(b + o_lutw) : dm.lut4;
   dm.luti8 = t.kqt ? reinterpret_cast<const uint32_t*>(b + o_luti8) : nullptr;
   dm.canon = canon ? reinterpret_cast<const uint32_t*>(b + o_canon) : nullptr;
   dm.tbase = reinterpret_cast<const uint32_t*>(b + o_tb);
@@ -395,15 +398,17 @@ bool make_resident(Model& M, Tensor& t, int threads) {
 }
 
 // Build and upload the device layout of a packed (fixed-rate) tensor: [symbol table 256 x 4 B, the payload bits of
-// decode_table4 for every symbol] padded to 256 B, then the symbols as 16-byte chunks [T][16 groups][64 rows]: chunk
-// (t, g, L) = symbols 16 g .. 16 g + 15 of tile row L, so a wave reads one group of its tile as 1 KB.
+// decode_table4 for every symbol; int8 table; the 16-token kernel's] padded to 256 B, then the symbols as 16-byte chunks
+// [T][16 groups][64 rows]: chunk (t, g, L) = symbols 16 g .. 16 g + 15 of tile row L, so a wave reads one group of its tile as 1 KB.
 bool make_resident_packed(Model& M, Tensor& t) {
   const int KS = t.KS(), NT = (int)(t.N / lw::TN), KT = KS / lw::TK, T = NT * KT;
   std::vector<uint8_t> blob((size_t)t.N * KS);
   if (!pread_all(M.fd, blob.data(), blob.size(), t.off)) return fail(t.name + ": read error");
-  const size_t o_words = 2 * 256 * 4, bytes = o_words + (size_t)T * lw::TN * lw::TK + 8 * 128;
+  const size_t o_words = 3 * 256 * 4, bytes = o_words + (size_t)T * lw::TN * lw::TK + 8 * 128;
   std::vector<uint8_t> host(bytes, 0);
-  if (t.kqt) {  // [symbol table 256 x 4 B][int8 symbol table 256 x 4 B]
+  uint64_t symbol_sum = 0;
+  for (const uint8_t v : blob) symbol_sum += v;
+  if (t.kqt) {  // [symbol table 256 x 4 B][int8 symbol table 256 x 4 B][lutw 256 x 4 B]
     std::vector<uint16_t> ident(lw::LUTN);
     for (int i = 0; i < lw::LUTN; ++i) ident[i] = (uint16_t)(i & 255);
     std::vector<uint32_t> tab(lw::LUTN);
@@ -411,9 +416,9 @@ bool make_resident_packed(Model& M, Tensor& t) {
     memcpy(host.data(), tab.data(), 256 * 4);
     lw::decode_table_i8(t.kqt, ident.data(), tab.data());
     memcpy(host.data() + 256 * 4, tab.data(), 256 * 4);
+    lw::decode_table4(t.kqt, ident.data(), tab.data(), mean_code(t, symbol_sum));
+    memcpy(host.data() + 2 * 256 * 4, tab.data(), 256 * 4);
   }
-  uint64_t symbol_sum = 0;
-  for (const uint8_t v : blob) symbol_sum += v;
   uint8_t* w = host.data() + o_words;
   for (int tr = 0; tr < NT; ++tr)
     for (int tc = 0; tc < KT; ++tc)
@@ -439,6 +444,7 @@ bool make_resident_packed(Model& M, Tensor& t) {
   uint8_t* b = static_cast<uint8_t*>(d);
   dm.lut4 = t.kqt ? reinterpret_cast<const uint32_t*>(b) : nullptr;
   dm.luti8 = t.kqt ? reinterpret_cast<const uint32_t*>(b + 256 * 4) : nullptr;
+  dm.lutw = t.kqt ? reinterpret_cast<const uint32_t*>(b + 2 * 256 * 4) : nullptr;
   dm.words = reinterpret_cast<const uint32_t*>(b + o_words);
   dm.packed = 1;
   dm.N = (int)t.N;

@@ -29,7 +29,7 @@
 // the mins with the sub-blocks' fp32 x sums, formed by launch_wide_x and held as three bf16 parts that add up to all 24
 // bits (as fp16 hi and lo a sum past 65504, 32 activations of 2047, would be infinite): parts in lane groups 0, 1 and 2 of
 // v_mfma_f32_16x16x32_bf16, the mins (at most 63) exact in bf16. Q5_K takes its mean code c
-// (DevMat::centre) off every code and with the sums instead: c d (sc . Sx), as exact, leaves products of sc (q - c), whose
+// (DevMat::centre, in its table) off every code and with the sums instead: c d (sc . Sx), as exact, leaves products of sc (q - c), whose
 // rounding counts for less.
 // Distance from 64 bits 1.3e-7 (2-norm), against 3e-6 of the ring kernel's fp16 dot products and 2e-7 .. 8e-7 of
 // k_fused_tiles_mma.
@@ -289,8 +289,7 @@ struct WideUnit {
       if constexpr (SYMB == 4 || (q & 1)) {  // 4 weights per lane
         constexpr int h = SYMB == 4 ? q & 1 : (q >> 1) & 1;
         auto scaled = [&](uint32_t w, h2v sv, h2v nv) {
-          h2v v = __builtin_bit_cast(h2v, w);
-          if constexpr (KQ == KQ_Q5_K) v -= dup((float)centre);
+          const h2v v = __builtin_bit_cast(h2v, w);
           return __builtin_bit_cast(uint32_t, KQ == KQ_IQ4_XS ? __builtin_elementwise_fma(v, sv, nv) : v * sv);
         };
 #pragma unroll
@@ -379,7 +378,7 @@ k_fused_wide(WidePlan plan, int buf_rows) {
           __builtin_amdgcn_global_load_lds(src + 64 * i, (__attribute__((address_space(3))) void*)(buf + 256 * i), 16, 0, 0);
     }
     {  // the decode table: 1 KB direct-to-LDS loads, chunk c by wave c mod W
-      const uint4* ta = reinterpret_cast<const uint4*>(e->M.lut4);
+      const uint4* ta = reinterpret_cast<const uint4*>(e->M.lutw);
       for (int c = wave; c < (PK ? 1 : 8); c += W)
         __builtin_amdgcn_global_load_lds(ta + 64 * c + lane, (__attribute__((address_space(3))) void*)(lut4 + 256 * c), 16,
                                          0, 0);
@@ -533,7 +532,7 @@ hipError_t launch_wide_x(WideXJobs q, hipStream_t s) {
 }
 
 bool wide_ok(const DevMat& M) {
-  return M.kqt >= KQ_Q4_K && M.kqt <= KQ_IQ4_XS && M.words && M.lut4 && M.side &&
+  return M.kqt >= KQ_Q4_K && M.kqt <= KQ_IQ4_XS && M.words && M.lutw && M.side &&
          (M.packed || (M.hsplit && M.rows && M.tbase && M.hrow && M.max_rows + 2 <= 256));
 }
 
